@@ -457,9 +457,12 @@ static int poisson_apply_strategy(dnsp_poisson* h) {
         const size_t N = (size_t)h->nx * h->nz * h->ny;
         DNSP_HIP_TRY(hipMalloc(&h->d_cp, sizeof(double) * N));
     }
-    // the blocked solve: compile-time x and z transforms, nx a multiple of 16,
-    // the partitioned tridiagonal; its workspace is one field
-    h->blk_ok = h->fft_strategy == DNSP_FFT_AUTO && h->ct_x && h->ct_z && xb_supported(h->nx) && part;
+    // the blocked solve: compile-time or register-direct x and z transforms,
+    // nx a multiple of 16, the partitioned tridiagonal; its workspace is one field
+    const bool rg = h->fft_strategy == DNSP_FFT_AUTO;
+    h->rx = rg && !h->ct_x ? rg_ops(h->nx) : nullptr;
+    h->rz = rg && !h->ct_z ? rg_ops(h->nz) : nullptr;
+    h->blk_ok = rg && rg_supported(h->nx) && rg_supported(h->nz) && h->nx % 16 == 0 && part;
     if (h->blk_ok && !h->d_W) {
         const size_t N = (size_t)h->nx * h->nz * h->ny;
         DNSP_HIP_TRY(hipMalloc(&h->d_W, sizeof(double) * N));
@@ -624,7 +627,8 @@ int dnsp_poisson_autotune(dnsp_poisson* h, double* work, int reps, void* stream,
             return DNSP_OK;
         };
         int* bk[5] = {&h->bxvar, &h->bzvar, &h->btvar, &h->bzvar_b, &h->bxvar_b};  // by stage
-        const int nv[5] = {kCtVariants, 2, kPartVariants, 2, kCtVariants};
+        const int nx_v = h->rx ? 1 : kCtVariants, nz_v = h->rz ? 1 : 2;  // register-direct: one shape
+        const int nv[5] = {nx_v, nz_v, kPartVariants, nz_v, nx_v};
         for (int stage = 0; stage < 5 && !rc; ++stage) {
             double bt = 1e30;
             int bv = *bk[stage];
@@ -714,10 +718,12 @@ int dnsp_poisson_stage(dnsp_poisson* h, const double* src, double* P, int stage,
     switch (stage) {
         case DNSP_STAGE_X_FWD:
             if (h->ct_x && x16) ct_x_launch(h->nx, h->xvar, false, src, P, nlines, h->d_twx, 1.0, st);
+            else if (h->rx) h->rx->xfwd(src, P, nlines, h->nz, (long)h->nx * h->nz, h->nx, 16, h->d_twx, st);
             else k_xfwd<<<gx, kFftThreads, ldsx, st>>>(src, P, h->nx, nlines, h->Gx, h->px);
             break;
         case DNSP_STAGE_Z_FWD:
             if (h->ct_z) ct_z_launch(h->nz, h->zvar, false, P, h->nx, h->ny, h->d_twz, st);
+            else if (h->rz) h->rz->zfwd(P, P, h->nx, h->ny, (long)h->nx * h->nz, 16, h->nx, 0, h->d_twz, st);
             else k_zfwd<<<gz, kFftThreads, ldsz, st>>>(P, h->nx, h->nz, h->ncol, h->TAz, h->pz);
             break;
         case DNSP_STAGE_TRIDIAG: {
@@ -734,10 +740,12 @@ int dnsp_poisson_stage(dnsp_poisson* h, const double* src, double* P, int stage,
         }
         case DNSP_STAGE_Z_BWD:
             if (h->ct_z) ct_z_launch(h->nz, h->zvar_b, true, P, h->nx, h->ny, h->d_twz, st);
+            else if (h->rz) h->rz->zbwd(P, P, h->nx, h->ny, (long)h->nx * h->nz, 16, h->nx, h->d_twz, st);
             else k_zbwd<<<gz, kFftThreads, ldsz, st>>>(P, h->nx, h->nz, h->ncol, h->TAz, h->pz);
             break;
         case DNSP_STAGE_X_BWD:
             if (h->ct_x && x16) ct_x_launch(h->nx, h->xvar_b, true, src, P, nlines, h->d_twx, inv_nxnz, st);
+            else if (h->rx) h->rx->xbwd(src, P, nlines, inv_nxnz, h->d_twx, st);
             else k_xbwd<<<gx, kFftThreads, ldsx, st>>>(src, P, h->nx, nlines, h->Gx, h->px, inv_nxnz);
             break;
         default:
@@ -786,18 +794,30 @@ int dnsp_poisson_solve_stage(dnsp_poisson* h, const double* rhs, double* P, int 
         return dnsp_poisson_stage(h, stage == 0 ? rhs : P, P, st_of[stage], stream);
     }
     hipStream_t st = as_stream(stream);
-    const long nlines = (long)h->nz * h->ny;
+    const long nlines = (long)h->nz * h->ny, plane = (long)h->nx * h->nz;
     const double inv_nxnz = 1.0 / ((double)h->nx * (double)h->nz + 0.0);
     // P lines -> W x-blocked -> P mode-major -> W x-blocked -> P lines -> P
     switch (stage) {
-        case 0: xb_x_launch(h->nx, h->bxvar, rhs, h->d_W, nlines, h->nz, h->d_twx, st); break;
-        case 1: mm_z_launch(h->nz, h->bzvar, false, h->d_W, P, h->nx, h->ny, h->d_twz, st); break;
+        case 0:
+            if (h->rx) h->rx->xfwd(rhs, h->d_W, nlines, h->nz, plane, 16, h->nz * 16, h->d_twx, st);
+            else xb_x_launch(h->nx, h->bxvar, rhs, h->d_W, nlines, h->nz, h->d_twx, st);
+            break;
+        case 1:
+            if (h->rz) h->rz->zfwd(h->d_W, P, h->nx, h->ny, plane, h->nz * 16, 16, 1, h->d_twz, st);
+            else mm_z_launch(h->nz, h->bzvar, false, h->d_W, P, h->nx, h->ny, h->d_twz, st);
+            break;
         case 2:
             part_launch<double, double, true>(h->btvar, P, h->d_ax, h->d_az, h->d_bands, h->nx, h->nz, h->ny,
                                               h->pcr_min, nullptr, nullptr, 0.0, st, nullptr, 0, h->d_W);
             break;
-        case 3: mm_z_launch(h->nz, h->bzvar_b, true, h->d_W, P, h->nx, h->ny, h->d_twz, st); break;
-        default: ct_x_launch(h->nx, h->bxvar_b, true, P, P, nlines, h->d_twx, inv_nxnz, st); break;
+        case 3:
+            if (h->rz) h->rz->zbwd(h->d_W, P, h->nx, h->ny, plane, h->nz * 16, 16, h->d_twz, st);
+            else mm_z_launch(h->nz, h->bzvar_b, true, h->d_W, P, h->nx, h->ny, h->d_twz, st);
+            break;
+        default:
+            if (h->rx) h->rx->xbwd(P, P, nlines, inv_nxnz, h->d_twx, st);
+            else ct_x_launch(h->nx, h->bxvar_b, true, P, P, nlines, h->d_twx, inv_nxnz, st);
+            break;
     }
     DNSP_LAUNCH_CHECK();
     return DNSP_OK;

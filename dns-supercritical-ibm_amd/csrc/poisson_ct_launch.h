@@ -16,11 +16,30 @@ void ct_z_launch(int n, int variant, bool inv, double* S, int nx, int ny, const 
 // to the x-blocked layout (variants as ct_x_launch); the z transforms from
 // x-blocked to mode-major (forward) and from x-blocked to halfcomplex lines
 // (inverse), variant 0: 256 threads, 1: 512.
-bool xb_supported(int n);
 void xb_x_launch(int n, int variant, const double* src, double* dst, long nlines, int nz, const double2* tw,
                  hipStream_t st);
 void mm_z_launch(int n, int variant, bool inv, const double* src, double* dst, int nx, int ny, const double2* tw,
                  hipStream_t st);
+// The FP64 transforms of every length 16..768 with prime factors up to 13
+// (poisson_reg.h; strides and layouts there).  z: mm = 1 writes the
+// mode-major blocks, 0 back in place.
+constexpr int kRgMin = 16, kRgMax = 768;
+constexpr bool rg_supported(int n) {
+    if (n < kRgMin || n > kRgMax) return false;
+    for (int p : {2, 3, 5, 7, 11, 13})
+        while (n % p == 0) n /= p;
+    return n == 1;
+}
+struct RgOps {
+    void (*xfwd)(const double* P, double* S, long nlines, int nz, long sk, int sj, int sb, const double2* tw,
+                 hipStream_t st);
+    void (*xbwd)(const double* S, double* P, long nlines, double scale, const double2* tw, hipStream_t st);
+    void (*zfwd)(const double* src, double* dst, int nx, int ny, long sk, int sc, int sj, int mm, const double2* tw,
+                 hipStream_t st);
+    void (*zbwd)(const double* src, double* dst, int nx, int ny, long sk, int sc, int sj, const double2* tw,
+                 hipStream_t st);
+};
+const RgOps* rg_ops(int n);  // NULL where not supported
 // FP32 z transforms; the forward one also turns the FP64 line sums lsum (if
 // not NULL) into the FP64 plane sums msum.
 void ct_z_launch(int n, int variant, bool inv, float* S, int nx, int ny, const float2* tw, const double* lsum,

@@ -47,8 +47,6 @@ static void ct_x_v(int v, bool inv, const double* src, double* dst, long nlines,
 
 #define DNSP_XB_SIZES(X) X(32) X(64) X(96) X(128) X(192) X(256) X(384) X(512) X(768)
 
-bool xb_supported(int n) { return ct_fft_supported(n) && n % 16 == 0; }
-
 void xb_x_launch(int n, int variant, const double* src, double* dst, long nlines, int nz, const double2* tw,
                  hipStream_t st) {
     switch (n) {

@@ -6,6 +6,7 @@
 
 #include "common.h"
 #include "fft_lds.h"
+#include "poisson_ct_launch.h"
 
 struct dnsp_poisson {
     int nx = 0, nz = 0, ny = 0;
@@ -25,6 +26,10 @@ struct dnsp_poisson {
     int fft_strategy = DNSP_FFT_AUTO;
     int tri_strategy = DNSP_TRIDIAG_AUTO;
     bool ct_x = false, ct_z = false;  // compile-time FFT kernels in use
+    // register-direct transforms (poisson_reg.h), where the length has no
+    // compile-time kernels with variants; NULL: not in use
+    const dnsp::RgOps* rx = nullptr;
+    const dnsp::RgOps* rz = nullptr;
     int xvar = 0, zvar = 0;           // their (tile, threads) variants, forward
     int xvar_b = 0, zvar_b = 0;       // and inverse transforms
     // blocked FP64 solve (x-blocked and mode-major layouts through d_W)
