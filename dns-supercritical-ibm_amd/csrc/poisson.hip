@@ -688,6 +688,7 @@ int dnsp_poisson_init(int nx_glob, int nz_glob, int ny, double inv_dx, double in
     h->inv_dx = inv_dx;
     h->inv_dz = inv_dz;
     h->precision = precision;
+    if (ny <= 32 * kPartChunks) h->tvar = h->btvar = part_default_variant(ny);
     int rc = poisson_setup(h, bands);
     if (!rc) rc = poisson_apply_strategy(h);
     if (!rc) rc = mixed_setup(h);

@@ -1020,15 +1020,18 @@ __device__ __forceinline__ long tri_group_mode(long grp, long ngroups, int M, in
     return grp * M + mi;
 }
 
-// The same groups for the mode-major blocks of the blocked solve (M = 16, nx
-// a multiple of 16), numbered z index first: group g in between holds x
-// block g / nz of z index g % nz, so that consecutive groups (which run side
-// by side on one XCD) read adjacent blocks and store adjacent 128-byte pieces.
+// The same groups for the mode-major blocks of the blocked solve (M = 8 or 16,
+// nx a multiple of 16), numbered z index first: the 16 / M groups of x block
+// ab and z index b follow those of b - 1, so that consecutive groups (which
+// run side by side on one XCD) read adjacent blocks and store adjacent pieces.
+template <int M>
 __device__ __forceinline__ long tri_group_mode_mm(long grp, long ngroups, int mi, int nx, int nz) {
-    if (grp == 0 || grp == ngroups) return tri_group_mode(grp, ngroups, 16, mi);
-    const unsigned g = (unsigned)grp;
+    static_assert(16 % M == 0, "groups within one 16-row block");
+    if (grp == 0 || grp == ngroups) return tri_group_mode(grp, ngroups, M, mi);
+    constexpr unsigned per = 16 / M;
+    const unsigned g = (unsigned)grp / per, sub = (unsigned)grp % per;
     const unsigned ab = g / (unsigned)nz, b = g - ab * (unsigned)nz;
-    return (long)ab * 16 + mi + (long)nx * b;
+    return (long)(ab * 16 + sub * M) + mi + (long)nx * b;
 }
 
 // Grid: tri_groups(plane, M) workgroups of M * P threads, 3 * MR * P values
@@ -1054,8 +1057,9 @@ __global__ __launch_bounds__(M * P, OCC) void kt_tri_part(T* S, const double* __
     // its own L2; workgroups reach XCDs round-robin)
     const int slot = xcd_tile((int)blockIdx.x, (int)gridDim.x);
     const long grp = glist ? (long)glist[slot] : (long)slot;
-    const long mode = MM && M == 16 ? tri_group_mode_mm(grp, plane / 16, mi, nx, nz)
-                                    : tri_group_mode(grp, (plane + M - 1) / M, M, mi);
+    long mode;
+    if constexpr (MM) mode = tri_group_mode_mm<M>(grp, plane / M, mi, nx, nz);
+    else mode = tri_group_mode(grp, (plane + M - 1) / M, M, mi);
     Ar d[MR];
     const double lam64 = tri_prologue<MR, P, M, T, Ar, MM>(d, smb, bands + (grp == 0 ? 3 * ny : 0), S, ax, az, mode,
                                                            plane, nx, ny, msum, nz);

@@ -46,21 +46,61 @@ void ct_z_launch(int n, int variant, bool inv, float* S, int nx, int ny, const f
                  double* msum, hipStream_t st);
 
 // Partitioned tridiagonal solve, ny <= 32 * kPartChunks.  Variants (P chunks
-// per mode of up to 32 rows, M modes per workgroup): 0 = P 32, M 16, registers
-// capped for 4 resident waves per SIMD; 1 = P 32, M 8; 2 = P 64, M 4;
-// 3 = P 64, M 8.
+// per mode of up to 32 rows, M modes per workgroup), FP64 spectra: 0 = P 32, M
+// 16, registers capped for 4 resident waves per SIMD; 1 = P 32, M 8; 2 = the
+// shape part_shape gives ny, with exactly ceil(ny / P) rows a chunk; 3 = P 16, M
+// 16 (ny <= 512, else P 64, M 8); 4..7 = the same with two-pass chunks.
 constexpr int kPartChunks = 32;
 constexpr int kPartVariants = 8;
 // tuner table: first slot of the x, z and tridiagonal variants of one form
 constexpr int kTuneSlot[3] = {0, 4, 8};
 constexpr int kTuneFormSlots = 16;
 int part_rows_for(int ny);  // rows per chunk at kPartChunks chunks (0: ny too large)
+// Chunks per mode by ny.  Fewer chunks shorten the reduced system (its
+// log2(P) barrier steps, and the serial sweep of the low modes) and move less
+// through LDS; more rows a chunk take more registers (about 6 VGPRs a row, 8 in
+// the two-pass form), hence fewer resident waves.  Measured per launch
+// (576 x 288 modes; us, fraction of 5.4 TB/s), against the 32 x 16 shape with
+// its rows rounded up to {2,3,4,6,8,12,16,24,32} that ran before:
+//   ny  33  P 4: 17.7 (0.92)  P 8: 18.9  P 16: 31.0  before 65
+//   ny  65  P 8: 29.2 (1.09)  P 4: 29.7  P 16: 35.5  before 66
+//   ny 129  P 16: 68.8 (0.92) P 8: 69.5              before 103
+//   ny 280  P 16: 146 (0.94)  P 32: 149              before 230 (384 rows)
+//   ny 384  P 16: 201 (0.94)  P 32: 203              before 247
+//   ny 770  P 32, M 8: 455 (0.83)  M 16: 555  P 16: 959  before 1403
+// Above 512 rows two workgroups of 16 modes no longer fit a CU's registers, so
+// a workgroup holds 8.
+struct PartShape {
+    int P, M, MR;
+};
+constexpr PartShape part_shape(int ny) {
+    const int P = ny <= 48 ? 4 : (ny <= 128 ? 8 : (ny <= 512 ? 16 : 32));
+    const int mr = (ny + P - 1) / P;
+    return {P, P == 32 ? 8 : 16, mr < 2 ? 2 : mr};
+}
+// The variant a handle starts with: part_shape's, two-pass from 21 rows a chunk
+// (at 24 rows 201 against 206 us, at 25 455 against 477; at 18 one-pass 146
+// against 149).
+constexpr int part_default_variant(int ny) { return part_shape(ny).MR > 20 ? 6 : 2; }
 // modes per workgroup (M) of a tridiagonal variant, FP32 or FP64 spectra
 int part_group_modes(int variant, int ny, bool fp32);
 // Ar: arithmetic type (double, or float for FP32 spectra); glist (device,
 // nlist entries): solve only the listed mode groups (NULL: all of them);
 // MM: S in the mode-major blocks of the blocked solve, the solution written
 // to So in its x-blocked layout.
+// The arguments of a rule-shaped FP64 launch (poisson_tri_rule_*.hip).
+struct PartArgs {
+    double* S;
+    const double *ax, *az, *bands;
+    int nx, nz, ny;
+    double pcr_min;
+    const double* msum;
+    double* pbar;
+    double inv_nxnz;
+    double* So;
+};
+template <bool TP, bool MM>
+void part_launch_rule(const PartArgs& a, hipStream_t st);
 template <typename T, typename Ar = double, bool MM = false>
 void part_launch(int variant, T* S, const double* ax, const double* az, const double* bands, int nx, int nz,
                  int ny, double pcr_min, const double* msum, double* pbar, double inv_nxnz, hipStream_t st,

@@ -89,17 +89,23 @@ void part_launch(int variant, T* S, const double* ax, const double* az, const do
     // FP64: 3 and 7 are (16, 16) for ny <= 512 (16 chunks of twice the
     // rows, one reduction step fewer), else (64, 8)
     const bool c16 = ny <= 16 * 32;
+    if constexpr (sizeof(T) == 8) {
+        if (variant == 2 || variant == 6) {
+            const PartArgs a{S, ax, az, bands, nx, nz, ny, pcr_min, msum, pbar, inv_nxnz, So};
+            if (variant == 2) part_launch_rule<false, MM>(a, st);
+            else part_launch_rule<true, MM>(a, st);
+            return;
+        }
+    }
     switch (variant) {
         case 0: DNSP_PV(32, 16, 4, false); break;
         case 1: DNSP_PV(32, 8, 1, false); break;
-        case 2: DNSP_PV(48, 16, 1, false); break;
         case 3:
             if (c16) DNSP_PV(16, 16, 1, false);
             else DNSP_PV(64, 8, 1, false);
             break;
         case 4: DNSP_PV(32, 16, 4, true); break;
         case 5: DNSP_PV(32, 8, 1, true); break;
-        case 6: DNSP_PV(48, 16, 1, true); break;
         default:
             if (c16) DNSP_PV(16, 16, 1, true);
             else DNSP_PV(64, 8, 1, true);

@@ -1,0 +1,4 @@
+// One-pass rule-shaped tridiagonal kernels, in place.
+#define DNSP_RULE_TP false
+#define DNSP_RULE_MM false
+#include "poisson_tri_rule.h"

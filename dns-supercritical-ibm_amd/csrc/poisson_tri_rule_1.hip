@@ -1,0 +1,4 @@
+// One-pass rule-shaped tridiagonal kernels, mode-major blocks.
+#define DNSP_RULE_TP false
+#define DNSP_RULE_MM true
+#include "poisson_tri_rule.h"

@@ -1,0 +1,4 @@
+// Two-pass rule-shaped tridiagonal kernels, in place.
+#define DNSP_RULE_TP true
+#define DNSP_RULE_MM false
+#include "poisson_tri_rule.h"
