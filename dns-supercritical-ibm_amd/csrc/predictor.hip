@@ -295,7 +295,7 @@ __device__ __forceinline__ void momentum_point(
 
 // U, V, W (and mu) are read at up to 16 neighbouring points each, so a
 // workgroup stages them in LDS (PlaneRing, stencil_grid.h): it owns a 64 x 4
-// (i, j) tile and marches through kRunK planes with planes k-1, k, k+1 of
+// (i, j) tile and marches through a run of planes with planes k-1, k, k+1 of
 // each field in a ring of three slots, the next plane's loads issued before
 // a step's arithmetic.  rho, div_now and buoyancy (four points each) are
 // read directly.  The per-thread version made 12.5 L1 and 2.9 L2 read
@@ -315,11 +315,7 @@ __global__ __launch_bounds__(kThreads) void k_momentum(
     const bool active = i < g.nx && j < g.nz;
     const double* fields[4] = {U, V, W, mu};
     PlaneRing<NF> ring(sF, fields, i0, j0, g.nx, g.nz);
-    ring.fetch(k0 - 1);
-    ring.put(k0 - 1);
-    ring.fetch(k0);
-    ring.put(k0);
-    ring.fetch(k0 + 1);
+    ring.prime(k0);
     const int e0 = ring_point();
     const long sz = g.sz(), sy = g.sy();
     // rho, div_now and buoy of this thread's column at plane k - 1: read at
@@ -640,7 +636,7 @@ __global__ __launch_bounds__(kThreads) void k_props(const double* __restrict__ T
 // RHS_energy and div_now = divjac RHS_energy at interior points
 // (mod_cfd_subroutines.f90:651-694), zero in rough-wall columns (:697-716).
 // T and cond are read at seven points each: a workgroup stages them in LDS
-// (PlaneRing, stencil_grid.h) and marches through kRunK planes of its 64 x 4
+// (PlaneRing, stencil_grid.h) and marches through a run of planes of its 64 x 4
 // tile, as k_momentum (at 384x256x192: 0.240 -> 0.230 ms; the per-thread
 // version served its 14 neighbour reads per point from L1 and L2), and
 // loads divjac one plane ahead (-> 0.212 ms).  Same expressions on the same
@@ -658,11 +654,7 @@ __global__ __launch_bounds__(kThreads) void k_rhs_energy(const double* __restric
     const bool active = i < g.nx && j < g.nz;
     const double* fields[2] = {T, cond};
     PlaneRing<2> ring(sF, fields, i0, j0, g.nx, g.nz);
-    ring.fetch(k0 - 1);
-    ring.put(k0 - 1);
-    ring.fetch(k0);
-    ring.put(k0);
-    ring.fetch(k0 + 1);
+    ring.prime(k0);
     const int e0 = ring_point();
     // the column's rough-wall slab (plane-independent) and divjac one plane
     // ahead, so that no step waits for a load of its own

@@ -98,7 +98,7 @@ __device__ __forceinline__ double rfac(double rho_min, double nb, double rc) {
 
 // Variable-density right-hand side.  P_now, P_old and rho are read at seven
 // points each, so they are staged in LDS: a workgroup owns a 64 x 4 (i, j)
-// tile and marches through a run of kRunK planes, keeping planes k-1, k,
+// tile and marches through a run of planes, keeping planes k-1, k,
 // k+1 of the three fields (tile plus one halo point in x and z) in a ring of
 // three LDS slots and loading one new plane per step (issued before the
 // step's arithmetic), so each of their values is read about once instead
@@ -119,11 +119,7 @@ __global__ __launch_bounds__(kTileX * kTileZ) void k_rhs_varprop(
     const long sz = h.sz(), sy = h.sy();
     const double* fields[3] = {Pn, Po, rho};
     PlaneRing<3> ring(sF, fields, i0, j0, h.nx, h.nz);
-    ring.fetch(k0 - 1);
-    ring.put(k0 - 1);
-    ring.fetch(k0);
-    ring.put(k0);
-    ring.fetch(k0 + 1);
+    ring.prime(k0);
     const double rho_min = *rho_min_p;
     const int e0 = ring_point();
     for (int k = k0; k < k1; ++k) {

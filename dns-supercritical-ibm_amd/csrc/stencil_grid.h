@@ -21,6 +21,7 @@ constexpr int kTileX = 64, kTileZ = 4;
 
 struct BandGrid {
     int nx, nz, nbx, hb, nbands, ny;
+    int run = 1;  // planes per workgroup
     __host__ __device__ int per_band() const { return nbx * hb * ny; }
     __host__ __device__ int blocks() const { return per_band() * nbands; }
 };
@@ -73,12 +74,26 @@ __device__ __forceinline__ bool band_point(const BandGrid& b, int& i, int& j, in
 // the next plane can be issued before a step's arithmetic.  Fields are the
 // reference's halo arrays ((nx+2)(nz+2)(ny+2), x fastest).
 constexpr int kRingX = kTileX + 2, kRingZ = kTileZ + 2, kRingP = kRingX * kRingZ;
-constexpr int kRunK = 16;  // planes per workgroup
 
-// Band order over tiles and runs of kRunK planes (an XCD walks the tiles of
-// its band one run at a time, so neighbouring tiles' halo rows meet in its
-// L2): launch ring_grid(nx, nz, ny).blocks() workgroups of band_block().
-inline BandGrid ring_grid(int nx, int nz, int ny) { return band_grid(nx, nz, (ny + kRunK - 1) / kRunK); }
+// Band order over tiles and runs of planes (an XCD walks the tiles of its band
+// one run at a time, so neighbouring tiles' halo rows meet in its L2): launch
+// ring_grid(nx, nz, ny).blocks() workgroups of band_block().  A run is 16
+// planes (it reads two more than it owns) where that leaves kRingBlocks
+// workgroups, else shorter: on a small grid a few long runs leave most of the
+// chip idle, each waiting for its own loads plane after plane.
+// (about three workgroups per CU are resident: 768 at once.  At 96 x 48 x 65 the
+// momentum, right-hand side and energy kernels took 45, 20 and 20 us in 120
+// workgroups of 16 planes; runs of 2 took the whole time step from 177 to 126
+// us.  Bounds of 1024 to 4096 differ by 1%.)
+constexpr int kRunK = 16, kRunMin = 2, kRingBlocks = 2048;
+inline BandGrid ring_grid(int nx, int nz, int ny) {
+    const BandGrid one = band_grid(nx, nz, 1);
+    int run = kRunK;
+    while (run > kRunMin && (long)one.blocks() * ((ny + run - 1) / run) < kRingBlocks) run /= 2;
+    BandGrid b = band_grid(nx, nz, (ny + run - 1) / run);
+    b.run = run;
+    return b;
+}
 
 // This workgroup's tile origin (i0, j0) and planes [k0, k1); false for a
 // workgroup past the last band's rows (uniform, before any barrier).
@@ -87,8 +102,8 @@ __device__ __forceinline__ bool ring_tile(const BandGrid& b, int ny, int& i0, in
     band_tile(b, bx, bz, run);
     i0 = bx * kTileX;
     j0 = bz * kTileZ;
-    k0 = run * kRunK;
-    k1 = k0 + kRunK < ny ? k0 + kRunK : ny;
+    k0 = run * b.run;
+    k1 = k0 + b.run < ny ? k0 + b.run : ny;
     return j0 < b.nz;
 }
 
@@ -129,6 +144,21 @@ struct PlaneRing {
         for (int u = 0; u < 2; ++u)
             if (ok[u])
                 for (int q = 0; q < NF; ++q) lds[q][slot][tid + u * kNT] = r[q][u];
+    }
+    // Planes k0 - 1 and k0 into their slots and k0 + 1 into the registers, the
+    // loads of all three in flight together.
+    __device__ __forceinline__ void prime(int k0) {
+        double a[2][NF][2];
+        for (int h = 0; h < 2; ++h)
+            for (int u = 0; u < 2; ++u)
+                for (int q = 0; q < NF; ++q) a[h][q][u] = ok[u] ? f[q][go[u] + (long)(k0 - 1 + h) * sy] : 0.0;
+        fetch(k0 + 1);
+        for (int h = 0; h < 2; ++h) {
+            const int slot = (k0 + 2 + h) % 3;
+            for (int u = 0; u < 2; ++u)
+                if (ok[u])
+                    for (int q = 0; q < NF; ++q) lds[q][slot][tid + u * kNT] = a[h][q][u];
+        }
     }
 };
 
