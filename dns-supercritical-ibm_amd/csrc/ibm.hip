@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "common.h"
+#include "halo_set.h"
 
 namespace dnsp {
 
@@ -53,6 +54,61 @@ __global__ void k_ibm_store(double* A, const long long* __restrict__ pos, const 
 __global__ void k_ibm_images(double* A, const long long* __restrict__ img, int m) {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r < m) A[img[2 * r]] = A[img[2 * r + 1]];
+}
+
+// The passes of up to four handles on up to four fields side by side: one launch
+// per pass instead of one per field and pass.  Blocks are numbered by field
+// (first[f]..first[f + 1]).
+struct ForceSet {
+    int n;
+    int first[5];
+    double* A[4];
+    const long long* pos[4];
+    const double* c[4];
+    int nrec[4];
+    const long long* img[4];
+    int nimg[4];
+    double wb[4], wt[4];
+};
+__device__ __forceinline__ int force_field(const ForceSet& s, int& b) {
+    int f = 0;
+    while (f + 1 < s.n && b >= s.first[f + 1]) ++f;
+    b -= s.first[f];
+    return f;
+}
+__global__ __launch_bounds__(kIbmThreads) void k_ibm_apply_set(ForceSet s) {
+#pragma clang fp contract(off)
+    int b = (int)blockIdx.x;
+    const int f = force_field(s, b);
+    const int r = b * kIbmThreads + (int)threadIdx.x;
+    if (r >= s.nrec[f]) return;
+    double* A = s.A[f];
+    const long long* pos = s.pos[f];
+    const double* c = s.c[f];
+    const double v = c[3 * r + 1] * A[pos[3 * r + 1]] + c[3 * r + 2] * A[pos[3 * r + 2]] + c[3 * r];
+    A[pos[3 * r]] = v;
+}
+// Images, and the planes k = -1 and ny of every field over the whole padded
+// plane: an image in one of those planes is overwritten by the wall value, so it
+// is left out and the two parts write different points.
+__global__ __launch_bounds__(kIbmThreads) void k_ibm_images_walls(ForceSet s, long pe, int ny, int wall_blocks) {
+    int b = (int)blockIdx.x;
+    const int f = force_field(s, b);
+    double* A = s.A[f];
+    if (b < 2 * wall_blocks) {
+        const bool up = b >= wall_blocks;
+        double* pl = A + (up ? (long)(ny + 1) * pe : 0);
+        const double v = up ? s.wt[f] : s.wb[f];
+        for (int u = 0; u < 4; ++u) {
+            const long o = ((long)(b - (up ? wall_blocks : 0)) * 4 + u) * kIbmThreads + threadIdx.x;
+            if (o < pe) pl[o] = v;
+        }
+        return;
+    }
+    const int r = (b - 2 * wall_blocks) * kIbmThreads + (int)threadIdx.x;
+    if (r >= s.nimg[f]) return;
+    const long long at = s.img[f][2 * r];
+    if (at >= pe && at < (ny + 1) * pe) A[at] = A[s.img[f][2 * r + 1]];
 }
 
 // ibm_part_2 (src/ibm_setup/mod_cfd_ibm.f90:47-141): column fills of a halo array
@@ -106,6 +162,57 @@ size_t ibm_device_bytes(const dnsp_ibm* h) {
     if (h->d_img) b += sizeof(long long) * 2 * (size_t)h->nimg;
     if (h->d_vals) b += sizeof(double) * (size_t)h->n;
     return b;
+}
+
+}  // namespace dnsp
+
+namespace dnsp {
+
+int ibm_force_walls(dnsp_ibm* const* hs, const HaloSet& s, int nx, int nz, int ny, hipStream_t st) {
+    // the shared launches take handles of this grid's halo arrays with disjoint
+    // targets and sources; otherwise the passes run field by field
+    bool shared = true;
+    for (int f = 0; f < s.n; ++f)
+        if (const dnsp_ibm* h = hs[f])
+            shared = shared && h->disjoint && h->nx == nx && h->nz == nz && h->ny == ny && h->nhalo + h->nskip == 1;
+    ForceSet fs{};
+    fs.n = s.n;
+    const long pe = (long)(nx + 2) * (nz + 2);
+    const int wall_blocks = (int)((pe + 4 * kIbmThreads - 1) / (4 * kIbmThreads));
+    int nrec = 0;
+    for (int f = 0; f < s.n; ++f) {
+        fs.A[f] = s.A[f];
+        fs.wb[f] = s.wb[f];
+        fs.wt[f] = s.wt[f];
+        fs.first[f] = nrec;
+        const dnsp_ibm* h = hs[f];
+        if (h && !shared) {
+            const int rc = dnsp_ibm_exec(hs[f], s.A[f], reinterpret_cast<void*>(st));
+            if (rc) return rc;
+        }
+        if (h && shared) {
+            fs.pos[f] = h->d_pos;
+            fs.c[f] = h->d_c;
+            fs.nrec[f] = h->n;
+            fs.img[f] = h->d_img;
+            fs.nimg[f] = h->nimg;
+            nrec += (h->n + kIbmThreads - 1) / kIbmThreads;
+        }
+    }
+    fs.first[s.n] = nrec;
+    if (nrec > 0) {
+        k_ibm_apply_set<<<nrec, kIbmThreads, 0, st>>>(fs);
+        DNSP_LAUNCH_CHECK();
+    }
+    int nb = 0;
+    for (int f = 0; f < s.n; ++f) {
+        fs.first[f] = nb;
+        nb += 2 * wall_blocks + (fs.nimg[f] + kIbmThreads - 1) / kIbmThreads;
+    }
+    fs.first[s.n] = nb;
+    k_ibm_images_walls<<<nb, kIbmThreads, 0, st>>>(fs, pe, ny, wall_blocks);
+    DNSP_LAUNCH_CHECK();
+    return DNSP_OK;
 }
 
 }  // namespace dnsp

@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "common.h"
+#include "halo_set.h"
 #include "stencil_grid.h"
 
 #pragma clang fp contract(off)
@@ -62,77 +63,7 @@ struct Phys {
 constexpr double kThird = 0.3333333333333333;
 constexpr double kTwoThirds = 0.6666666666666666;
 
-// --- periodicity and walls ---------------------------------------------------
-
-// cfd_periodicity on one rank for four fields: every padded plane gets its
-// periodic x/z halo, then the wall planes (A, C: k = -1 and ny; B: k = -1, 0
-// and ny) take the wall values over the whole padded plane.
-__global__ void k_periodicity4(double* A, double* B, double* C, double* T, Grid g, double ab, double bb, double cb,
-                               double tb, double at, double bt, double ct, double tt) {
-    const long pe = g.sy();
-    const long per_plane = 2L * (g.nz + 2) + 2L * g.nx;
-    const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long nwall = 9 * pe;
-    if (idx < nwall) {
-        const int which = (int)(idx / pe);
-        const long o = idx % pe;
-        const long top = (long)(g.ny + 1) * pe + o;
-        switch (which) {
-            case 0: A[o] = ab; break;
-            case 1: B[o] = bb; break;
-            case 2: B[pe + o] = bb; break;
-            case 3: C[o] = cb; break;
-            case 4: T[o] = tb; break;
-            case 5: A[top] = at; break;
-            case 6: B[top] = bt; break;
-            case 7: C[top] = ct; break;
-            default: T[top] = tt; break;
-        }
-        return;
-    }
-    const long r = idx - nwall;
-    if (r >= 4 * per_plane * g.ny) return;
-    const int f = (int)(r / (per_plane * g.ny));
-    const long rr = r % (per_plane * g.ny);
-    const int k = (int)(rr / per_plane);
-    const long s = rr % per_plane;
-    if (f == 1 && k == 0) return;  // B plane 0 is a wall plane
-    int i, j;
-    if (s < 2L * (g.nz + 2)) {
-        i = (s < g.nz + 2) ? -1 : g.nx;
-        j = (int)(s % (g.nz + 2)) - 1;
-    } else {
-        const long t = s - 2L * (g.nz + 2);
-        i = (int)(t % g.nx);
-        j = (t < g.nx) ? -1 : g.nz;
-    }
-    const int wi = i < 0 ? g.nx - 1 : (i >= g.nx ? 0 : i);
-    const int wj = j < 0 ? g.nz - 1 : (j >= g.nz ? 0 : j);
-    double* X = f == 0 ? A : (f == 1 ? B : (f == 2 ? C : T));
-    X[g.at(i, j, k)] = X[g.at(wi, wj, k)];
-}
-
-// Wall planes of ibm_part_1 (src/ibm_setup/mod_cfd_ibm.f90:26-38): k = -1
-// and ny of A, B, C, T over the whole padded plane (B bottom: k = -1 only).
-__global__ void k_walls4(double* A, double* B, double* C, double* T, Grid g, double ab, double bb, double cb,
-                         double tb, double at, double bt, double ct, double tt) {
-    const long pe = g.sy();
-    const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= 8 * pe) return;
-    const int which = (int)(idx / pe);
-    const long o = idx % pe;
-    const long top = (long)(g.ny + 1) * pe + o;
-    switch (which) {
-        case 0: A[o] = ab; break;
-        case 1: B[o] = bb; break;
-        case 2: C[o] = cb; break;
-        case 3: T[o] = tb; break;
-        case 4: A[top] = at; break;
-        case 5: B[top] = bt; break;
-        case 6: C[top] = ct; break;
-        default: T[top] = tt; break;
-    }
-}
+// --- div_now ghost planes and halos -------------------------------------------
 
 // div_now ghost planes by linear extrapolation of the first two interior
 // planes (mod_cfd_subroutines.f90:120-144), whole padded planes
@@ -1123,7 +1054,6 @@ int dnsp_predictor_enqueue(dnsp_predictor* pr, void* stream) {
     double* T = pr->f[DNSP_PRED_T];
     const double* wl = pr->walls;
     const long per_plane = 2L * (g.nz + 2) + 2L * g.nx;
-    const long nper = 9 * g.sy() + 4 * per_plane * g.ny;
     const BandGrid bg = band_grid(g.nx, g.nz, g.ny);
     const dim3 grid3((unsigned)bg.blocks());
     // tiles x runs of planes, for the kernels that stage planes in LDS
@@ -1136,44 +1066,37 @@ int dnsp_predictor_enqueue(dnsp_predictor* pr, void* stream) {
     void* vs = stream;
     double* F4[4] = {U, V, W, T};
     double* H4[4] = {Uh, Vh, Wh, T};
-    const double wb[4] = {wl[0], wl[1], wl[2], wl[3]}, wt[4] = {wl[4], wl[5], wl[6], wl[7]};
-    // ibm_part_2 (mod_cfd_ibm.f90:47-141) on four fields, each from its own slabs
-    auto fill_columns = [&](double* const* A4) {
-        int r = DNSP_OK;
-        for (int c = 0; c < 4 && !r; ++c)
-            if (pr->d_bot[c])
-                r = dnsp_ibm_part2(A4[c], pr->d_bot[c], pr->d_top[c], g.nx, g.nz, g.ny, c == 1 ? g.ny : g.ny - 1,
-                                   wb[c], wt[c], vs);
-        return r;
+    // the fields of A4 with their walls and, with columns, their slabs
+    auto field_set = [&](double* const* A4, bool with_columns) {
+        HaloSet hs;
+        hs.n = 4;
+        hs.v = 1;
+        for (int c = 0; c < 4; ++c) {
+            hs.A[c] = A4[c];
+            hs.wb[c] = wl[c];
+            hs.wt[c] = wl[4 + c];
+            hs.bot[c] = with_columns ? pr->d_bot[c] : nullptr;
+            hs.top[c] = with_columns ? pr->d_top[c] : nullptr;
+        }
+        return hs;
     };
     // ibm_part_1 (mod_cfd_ibm.f90:10-45): forcing of four fields, their wall
     // planes, and (force_div) the forcing of div_now
     auto part_1 = [&](double* const* A4, bool force_div) {
-        int r = DNSP_OK;
-        for (int c = 0; c < 4 && !r; ++c)
-            if (pr->ibm[c]) r = dnsp_ibm_exec(pr->ibm[c], A4[c], vs);
-        if (r) return r;
-        k_walls4<<<blocks_for(8 * g.sy()), kThreads, 0, st>>>(A4[0], A4[1], A4[2], A4[3], g, wl[0], wl[1], wl[2],
-                                                              wl[3], wl[4], wl[5], wl[6], wl[7]);
-        if (force_div && pr->ibm[4]) r = dnsp_ibm_exec(pr->ibm[4], dvn, vs);
+        int r = ibm_force_walls(pr->ibm, field_set(A4, false), g.nx, g.nz, g.ny, st);
+        if (!r && force_div && pr->ibm[4]) r = dnsp_ibm_exec(pr->ibm[4], dvn, vs);
         return r;
     };
     if (!rough) {
         // 1. cfd_periodicity(U, V, W, T)
-        k_periodicity4<<<blocks_for(nper), kThreads, 0, st>>>(U, V, W, T, g, wl[0], wl[1], wl[2], wl[3], wl[4],
-                                                              wl[5], wl[6], wl[7]);
+        rc = halo_columns_periodicity(field_set(F4, false), g.nx, g.nz, g.ny, st);
     } else {
         // 1. rough walls (mod_cfd_subroutines.f90:98-108): with quady the columns
         // of U, V, W, T and cfd_periodicity first; then ibm_part_1
-        if (pr->quady) {
-            rc = fill_columns(F4);
-            if (rc) return rc;
-            k_periodicity4<<<blocks_for(nper), kThreads, 0, st>>>(U, V, W, T, g, wl[0], wl[1], wl[2], wl[3], wl[4],
-                                                                  wl[5], wl[6], wl[7]);
-        }
-        rc = part_1(F4, vp);
-        if (rc) return rc;
+        if (pr->quady) rc = halo_columns_periodicity(field_set(F4, true), g.nx, g.nz, g.ny, st);
+        if (!rc) rc = part_1(F4, vp);
     }
+    if (rc) return rc;
     // 2. div_now ghost planes
     if (vp)
         k_div_walls<<<blocks_for(2 * g.sy()), kThreads, 0, st>>>(dvn, g, pr->extrap[0], pr->extrap[1],
@@ -1198,16 +1121,12 @@ int dnsp_predictor_enqueue(dnsp_predictor* pr, void* stream) {
         k_temp_rhs<false><<<grid3, blk3, 0, st>>>(T, U, V, W, nullptr, nullptr, nullptr, pr->d_rt_now, g, bg, pr->G,
                                                       pr->p);
     k_temp_update<<<grid3, blk3, 0, st>>>(T, pr->d_rt_now, pr->f[DNSP_PRED_RT_OLD], g, bg, pr->p.dt);
-    // 5. rough walls: columns of the hats and T, each from its own slabs
-    if (columns) {
-        rc = fill_columns(H4);
-        if (rc) return rc;
-    }
+    // 5. rough walls: columns of the hats and T, each from its own slabs;
     // periodicity of the hats and T with their wall planes (with rough walls
     // the reference sets only the halos the right-hand side reads, V_hat's
     // walls and T's; the extra halo and wall values are read by nothing)
-    k_periodicity4<<<blocks_for(nper), kThreads, 0, st>>>(Uh, Vh, Wh, T, g, wl[0], wl[1], wl[2], wl[3], wl[4],
-                                                          wl[5], wl[6], wl[7]);
+    rc = halo_columns_periodicity(field_set(H4, true), g.nx, g.nz, g.ny, st);
+    if (rc) return rc;
     if (rough && pr->quady) {
         // quady (mod_cfd_subroutines.f90:417-427): ibm_part_1 on the hats and T;
         // its last argument (.false.) leaves the div_now forcing on; then T's halos

@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "common.h"
+#include "halo_set.h"
 #include "stencil_grid.h"
 
 namespace dnsp {
@@ -172,44 +173,84 @@ __global__ void k_min_init(double* out) {
         *reinterpret_cast<unsigned long long*>(out) = 0xffffffffffffffffull;
 }
 
-// Workgroups stride over groups of kMinRows interior x rows; a group's
-// kMinRows * nx values are spread over all the workgroup's threads (whole
-// rows per thread left half the lanes idle at nx = 384), and each thread
-// issues kMinLoads loads before comparing their keys.
-constexpr int kMinRows = 8, kMinLoads = 4;
-__global__ void k_min_interior(const double* __restrict__ A, Halo h, double* out) {
-    __shared__ unsigned long long red[kStencilThreads];
-    const int rows = h.nz * h.ny;
-    const int per = kMinRows * h.nx;
-    unsigned long long best = 0xffffffffffffffffull;
-    for (int row0 = (int)blockIdx.x * kMinRows; row0 < rows; row0 += (int)gridDim.x * kMinRows) {
-        for (int e0 = (int)threadIdx.x; e0 < per; e0 += kMinLoads * kStencilThreads) {
-            double v[kMinLoads];
-#pragma unroll
-            for (int u = 0; u < kMinLoads; ++u) {
-                const int e = e0 + u * kStencilThreads;
-                const int r = (int)((unsigned)e / (unsigned)h.nx);
-                const int i = e - r * h.nx;
-                const int row = row0 + r;
-                const int k = row / h.nz, j = row - k * h.nz;
-                // past the group or the last row: a repeat of an interior value
-                const long at = e < per && row < rows ? h.at(i, j, k) : h.at(0, 0, 0);
-                v[u] = A[at];
-            }
-#pragma unroll
-            for (int u = 0; u < kMinLoads; ++u) {
-                const unsigned long long key = dkey(v[u]);
-                best = key < best ? key : best;
-            }
+// Minimum key of this thread's share of the interior: the grid strides over the
+// padded planes 0..ny-1 (workgroups side by side on adjacent memory), kMinLoads
+// coalesced loads in flight per thread; halo points are masked by their row
+// and column, which advance by additions (one division per thread and stride,
+// none per point).
+constexpr int kMinLoads = 8;
+__device__ __forceinline__ unsigned long long min_key_range(const double* __restrict__ A, const Halo& h) {
+    const unsigned px = (unsigned)h.nx + 2, pz = (unsigned)h.nz + 2;
+    const long n = (long)h.ny * h.sy();  // plane 0 starts at element sy
+    constexpr int per = kMinLoads * kStencilThreads;
+    const double* src = A + h.sy();
+    // column and row advance of one load, and of the rest of a grid stride
+    const unsigned dr = kStencilThreads / px, dc = kStencilThreads - dr * px, drz = dr % pz;
+    const unsigned skip = (gridDim.x - 1) * (unsigned)per, sr = skip / px, sc = skip - sr * px, srz = sr % pz;
+    long e = (long)blockIdx.x * per + (long)threadIdx.x;
+    const long row = e / px;
+    unsigned c = (unsigned)(e - row * px), r = (unsigned)(row % pz);
+    auto advance = [&](unsigned ac, unsigned ar) {
+        c += ac;
+        r += ar;
+        if (c >= px) {
+            c -= px;
+            ++r;
         }
+        r = r >= pz ? r - pz : r;
+    };
+    unsigned long long best = 0xffffffffffffffffull;
+    for (; e < n; e += (long)gridDim.x * per) {
+        double v[kMinLoads];
+#pragma unroll
+        for (int u = 0; u < kMinLoads; ++u) {
+            const long at = e + (long)u * kStencilThreads;
+            v[u] = src[at < n ? at : e];
+        }
+#pragma unroll
+        for (int u = 0; u < kMinLoads; ++u) {
+            const bool in = e + (long)u * kStencilThreads < n && c >= 1 && c <= (unsigned)h.nx && r >= 1 &&
+                            r <= (unsigned)h.nz;
+            const unsigned long long key = dkey(v[u]);
+            best = in && key < best ? key : best;
+            advance(dc, drz);
+        }
+        advance(sc, srz);
     }
+    return best;
+}
+
+// Minimum over the workgroup, in thread 0.
+__device__ __forceinline__ unsigned long long min_key_block(unsigned long long best, unsigned long long* red) {
     red[threadIdx.x] = best;
     __syncthreads();
     for (int s = kStencilThreads / 2; s > 0; s >>= 1) {
         if ((int)threadIdx.x < s && red[threadIdx.x + s] < red[threadIdx.x]) red[threadIdx.x] = red[threadIdx.x + s];
         __syncthreads();
     }
-    if (threadIdx.x == 0) atomicMin(reinterpret_cast<unsigned long long*>(out), red[0]);
+    return red[0];
+}
+
+__global__ __launch_bounds__(kStencilThreads) void k_min_interior(const double* __restrict__ A, Halo h, double* out) {
+    __shared__ unsigned long long red[kStencilThreads];
+    const unsigned long long m = min_key_block(min_key_range(A, h), red);
+    if (threadIdx.x == 0) atomicMin(reinterpret_cast<unsigned long long*>(out), m);
+}
+
+// The same with one key per workgroup in part, then one workgroup over them.
+__global__ __launch_bounds__(kStencilThreads) void k_min_partial(const double* __restrict__ A, Halo h,
+                                                                 unsigned long long* __restrict__ part) {
+    __shared__ unsigned long long red[kStencilThreads];
+    const unsigned long long m = min_key_block(min_key_range(A, h), red);
+    if (threadIdx.x == 0) part[blockIdx.x] = m;
+}
+__global__ __launch_bounds__(kStencilThreads) void k_min_final(const unsigned long long* __restrict__ part, int n,
+                                                               double* out) {
+    __shared__ unsigned long long red[kStencilThreads];
+    unsigned long long best = 0xffffffffffffffffull;
+    for (int i = (int)threadIdx.x; i < n; i += kStencilThreads) best = part[i] < best ? part[i] : best;
+    const unsigned long long m = min_key_block(best, red);
+    if (threadIdx.x == 0) *out = dunkey(m);
 }
 
 __global__ void k_min_decode(double* out) {
@@ -304,55 +345,137 @@ __global__ void k_pper_rotate(const double* __restrict__ P, double* P_per, doubl
     }
 }
 
-// Velocity halos and wall planes after the correction (update_vars :1225-1244):
-// ghost planes k = -1, ny (and k = 0 for V) take the wall values over the whole
-// padded plane; other planes get periodic x/z halos.
-__global__ void k_vel_finish(double* U, double* V, double* W, Halo h, double ub, double vb, double wb, double ut,
-                             double vt, double wt) {
-    const long pe = h.sy();
-    const long per_plane = 2L * (h.nz + 2) + 2L * h.nx;
-    const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    // part 1: wall planes: U,W at k=-1,ny ; V at k=-1,0,ny
-    const long nwall = 7 * pe;
-    if (idx < nwall) {
-        const int which = (int)(idx / pe);
-        const long o = idx % pe;
-        switch (which) {
-            case 0: U[o] = ub; break;
-            case 1: W[o] = wb; break;
-            case 2: V[o] = vb; break;
-            case 3: V[pe + o] = vb; break;
-            case 4: U[(long)(h.ny + 1) * pe + o] = ut; break;
-            case 5: W[(long)(h.ny + 1) * pe + o] = wt; break;
-            default: V[(long)(h.ny + 1) * pe + o] = vt; break;
-        }
+// Columns, periodic halos and wall planes of a HaloSet.  Blocks are numbered per
+// field: CB over the columns, ny PB over the halo points of planes 0..ny-1, then
+// 3 WB over the wall planes -1, ny and (V) 0; the block's part and plane are
+// workgroup-uniform.  Every point has one writer: columns leave the wall
+// planes out, and a halo point whose image lies in a column takes the column's
+// value instead of reading it.
+constexpr int kWallElems = 4 * kStencilThreads;  // wall-plane points per block
+struct SetGrid {
+    int CB, PB, WB;
+    __host__ __device__ int per_field(int ny) const { return CB + ny * PB + 3 * WB; }
+};
+
+__global__ __launch_bounds__(kStencilThreads) void k_halo_set(HaloSet s, Halo h, SetGrid sg) {
+    const int per = sg.per_field(h.ny);
+    const int f = (int)blockIdx.x / per;
+    int b = (int)blockIdx.x - f * per;
+    double* A = s.A[f];
+    const int* bot = s.bot[f];
+    const int* top = s.top[f];
+    const double wb = s.dw ? s.dw[f] : s.wb[f], wt = s.dw ? s.dw[s.n + f] : s.wt[f];
+    const int k0 = f == s.v ? 1 : 0;  // first plane that is not a wall plane
+    const int tid = (int)threadIdx.x;
+    if (b < sg.CB) {
+        const int col = b * kStencilThreads + tid;
+        if (bot == nullptr || col >= h.nx * h.nz) return;
+        const int j = col / h.nx, i = col - j * h.nx;
+        const int cb = bot[col], ct = top[col];
+        const int t0 = ct > k0 ? ct : k0;
+        double* c = A + h.at(i, j, 0);
+        for (int k = k0; k <= cb && k < t0 && k < h.ny; ++k) c[k * h.sy()] = wb;
+        for (int k = t0; k < h.ny; ++k) c[k * h.sy()] = wt;
         return;
     }
-    // part 2: periodic halos of planes k = 0..ny-1 (U, W) and 1..ny-1 (V)
-    const long r = idx - nwall;
-    if (r >= 3 * per_plane * h.ny) return;
-    const int f = (int)(r / (per_plane * h.ny));
-    const long rr = r % (per_plane * h.ny);
-    const int k = (int)(rr / per_plane);
-    const long s = rr % per_plane;
-    if (f == 1 && k == 0) return;  // V plane 0 is a wall plane
-    int i, j;
-    if (s < 2L * (h.nz + 2)) {
-        i = (s < h.nz + 2) ? -1 : h.nx;
-        j = (int)(s % (h.nz + 2)) - 1;
-    } else {
-        const long t = s - 2L * (h.nz + 2);
-        i = (int)(t % h.nx);
-        j = (t < h.nx) ? -1 : h.nz;
+    b -= sg.CB;
+    if (b < h.ny * sg.PB) {
+        const int k = b / sg.PB;
+        const int e = (b - k * sg.PB) * kStencilThreads + tid;
+        const int pz = h.nz + 2;
+        if (k < k0 || e >= 2 * pz + 2 * h.nx) return;
+        int i, j;
+        if (e < 2 * pz) {
+            i = e < pz ? -1 : h.nx;
+            j = (e < pz ? e : e - pz) - 1;
+        } else {
+            const int t = e - 2 * pz;
+            i = t < h.nx ? t : t - h.nx;
+            j = t < h.nx ? -1 : h.nz;
+        }
+        const int wi = i < 0 ? h.nx - 1 : (i >= h.nx ? 0 : i);
+        const int wj = j < 0 ? h.nz - 1 : (j >= h.nz ? 0 : j);
+        double v;
+        bool column = false;
+        if (bot != nullptr) {
+            const int col = wi + h.nx * wj;
+            const bool up = k >= top[col];
+            column = up || k <= bot[col];
+            v = up ? wt : wb;
+        }
+        if (!column) v = A[h.at(wi, wj, k)];
+        A[h.at(i, j, k)] = v;
+        return;
     }
-    const int wi = i < 0 ? h.nx - 1 : (i >= h.nx ? 0 : i);
-    const int wj = j < 0 ? h.nz - 1 : (j >= h.nz ? 0 : j);
-    double* A = f == 0 ? U : (f == 1 ? V : W);
-    A[h.at(i, j, k)] = A[h.at(wi, wj, k)];
+    b -= h.ny * sg.PB;
+    const int w = b / sg.WB;  // 0: plane -1, 1: plane ny, 2: plane 0 (V)
+    if (w == 2 && f != s.v) return;
+    const int pe = (int)h.sy();
+    double* pl = A + (long)(w == 0 ? 0 : (w == 1 ? h.ny + 1 : 1)) * pe;
+    const double val = w == 1 ? wt : wb;
+    for (int u = 0; u < 4; ++u) {
+        const int o = (b - w * sg.WB) * kWallElems + u * kStencilThreads + tid;
+        if (o < pe) pl[o] = val;
+    }
+}
+
+static int launch_halo_set(const HaloSet& s, const Halo& h, hipStream_t st) {
+    bool columns = false;
+    for (int f = 0; f < s.n; ++f) columns = columns || s.bot[f];
+    SetGrid sg;
+    sg.CB = columns ? blocks_for((long)h.nx * h.nz) : 0;
+    sg.PB = blocks_for(2L * (h.nz + 2) + 2L * h.nx);
+    sg.WB = blocks_for(h.sy(), kWallElems);
+    k_halo_set<<<s.n * sg.per_field(h.ny), kStencilThreads, 0, st>>>(s, h, sg);
+    DNSP_LAUNCH_CHECK();
+    return DNSP_OK;
+}
+
+// Workgroups of the minimum: one range of kMinLoads loads per thread at least,
+// at most kMinBlocks (four per CU).
+static int min_blocks(const Halo& h) {
+    const long n = (long)h.ny * h.sy(), per = (long)kMinLoads * kStencilThreads;
+    return (int)std::min((long)kMinBlocks, (n + per - 1) / per);
 }
 
 static bool halo_ok(int nx, int nz, int ny) {
     return nx >= 1 && nz >= 1 && ny >= 1 && (double)(nx + 2) * (nz + 2) * (ny + 2) < 4e12;
+}
+
+int halo_columns_periodicity(const HaloSet& s, int nx, int nz, int ny, hipStream_t st) {
+    return launch_halo_set(s, Halo{nx, nz, ny}, st);
+}
+
+int rho_min_scratch(const double* rho, int nx, int nz, int ny, double* out, double* scratch, hipStream_t st) {
+    const Halo h{nx, nz, ny};
+    const int nb = min_blocks(h);
+    auto* part = reinterpret_cast<unsigned long long*>(scratch);
+    k_min_partial<<<nb, kStencilThreads, 0, st>>>(rho, h, part);
+    k_min_final<<<1, kStencilThreads, 0, st>>>(part, nb, out);
+    DNSP_LAUNCH_CHECK();
+    return DNSP_OK;
+}
+
+int update_vars_interior(const double* P, double* P_per, double* P_now, double* P_old, double* U, double* V, double* W,
+                         const double* U_hat, const double* V_hat, const double* W_hat, const double* rho,
+                         const double* hi, const double* lo, const double* rho_min, int nx, int nz, int ny,
+                         int kmin_Vhat, double dtmax, double inv_dx, double inv_dz, int use_incompressible,
+                         hipStream_t st) {
+    const Halo h{nx, nz, ny};
+    const BandGrid bg = band_grid(nx, nz, ny);
+    if (use_incompressible)
+        k_update_incomp<<<bg.blocks(), band_block(), 0, st>>>(P, U, V, W, U_hat, V_hat, W_hat, hi, lo, h, bg,
+                                                              kmin_Vhat, dtmax, inv_dx, inv_dz);
+    else
+        k_update_varprop<<<bg.blocks(), band_block(), 0, st>>>(P, U, V, W, U_hat, V_hat, W_hat, P_now, P_old, rho, hi,
+                                                               lo, rho_min, h, bg, kmin_Vhat, dtmax, inv_dx, inv_dz);
+    DNSP_LAUNCH_CHECK();
+    if (P_per || !use_incompressible) {
+        auto kr = h.total() < (1L << 31) ? k_pper_rotate<true> : k_pper_rotate<false>;
+        kr<<<blocks_for(h.total()), kStencilThreads, 0, st>>>(P, P_per, P_now, P_old, h, use_incompressible ? 0 : 1);
+        DNSP_LAUNCH_CHECK();
+    }
+    return DNSP_OK;
 }
 
 }  // namespace dnsp
@@ -431,7 +554,7 @@ int dnsp_rho_min(const double* rho, int nx, int nz, int ny, double* out, void* s
     DNSP_ARG_CHECK(rho && out && halo_ok(nx, nz, ny), "invalid arguments");
     Halo h{nx, nz, ny};
     hipStream_t st = as_stream(stream);
-    const int nb = std::min(2048, (nz * ny + kMinRows - 1) / kMinRows);
+    const int nb = min_blocks(h);
     k_min_init<<<1, 1, 0, st>>>(out);
     k_min_interior<<<nb, kStencilThreads, 0, st>>>(rho, h, out);
     k_min_decode<<<1, 1, 0, st>>>(out);
@@ -451,27 +574,17 @@ int dnsp_update_vars(const double* P, double* P_per, double* P_now, double* P_ol
     DNSP_ARG_CHECK(kmin_Vhat >= 0 && kmin_Vhat <= ny, "kmin_Vhat=%d", kmin_Vhat);
     DNSP_ARG_CHECK(use_incompressible || (P_now && P_old && rho && rho_min),
                    "variable-density correction needs P_now, P_old, rho and rho_min");
-    Halo h{nx, nz, ny};
-    hipStream_t st = as_stream(stream);
-    const BandGrid bg = band_grid(nx, nz, ny);
-    if (use_incompressible)
-        k_update_incomp<<<bg.blocks(), band_block(), 0, st>>>(P, U, V, W, U_hat, V_hat, W_hat, dPdy_ddy_hi,
-                                                              dPdy_ddy_lo, h, bg, kmin_Vhat, dtmax, inv_dx, inv_dz);
-    else
-        k_update_varprop<<<bg.blocks(), band_block(), 0, st>>>(P, U, V, W, U_hat, V_hat, W_hat, P_now, P_old, rho,
-                                                               dPdy_ddy_hi, dPdy_ddy_lo, rho_min, h, bg, kmin_Vhat,
-                                                               dtmax, inv_dx, inv_dz);
-    DNSP_LAUNCH_CHECK();
-    if (P_per || !use_incompressible) {
-        auto kr = h.total() < (1L << 31) ? k_pper_rotate<true> : k_pper_rotate<false>;
-        kr<<<blocks_for(h.total()), kStencilThreads, 0, st>>>(P, P_per, P_now, P_old, h, use_incompressible ? 0 : 1);
-        DNSP_LAUNCH_CHECK();
-    }
-    const long nfin = 7 * h.sy() + 3 * (2L * (nz + 2) + 2L * nx) * ny;
-    k_vel_finish<<<blocks_for(nfin), kStencilThreads, 0, st>>>(U, V, W, h, wall_bc[0], wall_bc[1], wall_bc[2],
-                                                              wall_bc[3], wall_bc[4], wall_bc[5]);
-    DNSP_LAUNCH_CHECK();
-    return DNSP_OK;
+    const int rc = update_vars_interior(P, P_per, P_now, P_old, U, V, W, U_hat, V_hat, W_hat, rho, dPdy_ddy_hi,
+                                        dPdy_ddy_lo, rho_min, nx, nz, ny, kmin_Vhat, dtmax, inv_dx, inv_dz,
+                                        use_incompressible, as_stream(stream));
+    if (rc) return rc;
+    HaloSet hs;
+    hs.n = 3;
+    hs.v = 1;
+    double* const A[3] = {U, V, W};
+    for (int f = 0; f < 3; ++f) hs.A[f] = A[f];
+    hs.dw = wall_bc;
+    return halo_columns_periodicity(hs, nx, nz, ny, as_stream(stream));
 }
 
 // calc_bands.py:272-277 and :336-343 (rows 0..ny-1 of dPdy_ddy_lh, as read at

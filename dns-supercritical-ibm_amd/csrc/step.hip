@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "common.h"
+#include "halo_set.h"
 
 using namespace dnsp;
 
@@ -77,7 +78,8 @@ int enqueue(dnsp_step* s, int refinements, hipStream_t st) {
         rc = dnsp_build_p_rhs(P, F[DNSP_STEP_U_HAT], F[DNSP_STEP_W_HAT], F[DNSP_STEP_V_HAT], inv_dy_p, nx, nz, ny,
                               1.0 / s->dtmax, s->inv_dx, s->inv_dz, vs);
     } else {
-        rc = dnsp_rho_min(F[DNSP_STEP_RHO], nx, nz, ny, s->d_rho_min, vs);
+        // P, not yet written by the right-hand side, is the minimum's scratch
+        rc = rho_min_scratch(F[DNSP_STEP_RHO], nx, nz, ny, s->d_rho_min, P, st);
         if (!rc)
             rc = dnsp_build_p_rhs_varprop(P, F[DNSP_STEP_U_HAT], F[DNSP_STEP_W_HAT], F[DNSP_STEP_V_HAT],
                                           F[DNSP_STEP_P_NOW], F[DNSP_STEP_P_OLD], F[DNSP_STEP_RHO],
@@ -88,46 +90,33 @@ int enqueue(dnsp_step* s, int refinements, hipStream_t st) {
     if (rc) return rc;
     rc = refinements < 0 ? dnsp_poisson_run(s->poisson, P, vs) : dnsp_poisson_run_mixed(s->poisson, P, refinements, vs);
     if (rc) return rc;
-    rc = dnsp_update_vars(P, F[DNSP_STEP_P_PER], F[DNSP_STEP_P_NOW], F[DNSP_STEP_P_OLD], F[DNSP_STEP_U],
-                          F[DNSP_STEP_V], F[DNSP_STEP_W], F[DNSP_STEP_U_HAT], F[DNSP_STEP_V_HAT], F[DNSP_STEP_W_HAT],
-                          F[DNSP_STEP_RHO], hi, lo, s->d_rho_min, s->d_walls, nx, nz, ny, 1, s->dtmax, s->inv_dx,
-                          s->inv_dz, s->incompressible, vs);
+    rc = update_vars_interior(P, F[DNSP_STEP_P_PER], F[DNSP_STEP_P_NOW], F[DNSP_STEP_P_OLD], F[DNSP_STEP_U],
+                              F[DNSP_STEP_V], F[DNSP_STEP_W], F[DNSP_STEP_U_HAT], F[DNSP_STEP_V_HAT],
+                              F[DNSP_STEP_W_HAT], F[DNSP_STEP_RHO], hi, lo, s->d_rho_min, nx, nz, ny, 1, s->dtmax,
+                              s->inv_dx, s->inv_dz, s->incompressible, st);
     if (rc) return rc;
-    // Rough walls: the opening of the next build_vars on U, V, W
-    // (mod_cfd_subroutines.f90:98-113), so the step ends on the velocities the
-    // next predictor reads.  With column slabs (the quadratic-wall ordering,
-    // use_rough_surf_quady) ibm_part_2 fills each component's columns and
-    // cfd_periodicity restores halos and walls first; then ibm_part_1 forces
-    // U, V, W and sets their wall ghost planes (mod_cfd_ibm.f90:26-38).  The
-    // forcing comes last, so no column fill overwrites a forced value.
+    // update_vars' halos and wall planes.  Rough walls: the opening of the next
+    // build_vars on U, V, W (mod_cfd_subroutines.f90:98-113), so the step ends
+    // on the velocities the next predictor reads.  With column slabs (the
+    // quadratic-wall ordering, use_rough_surf_quady) ibm_part_2 fills each
+    // component's columns and cfd_periodicity restores halos and walls, in the
+    // same launch: both write what update_vars' own halos would.  Then
+    // ibm_part_1 forces U, V, W and sets their wall ghost planes
+    // (mod_cfd_ibm.f90:26-38).  The forcing comes last, so no column fill
+    // overwrites a forced value.
+    HaloSet hs;
+    hs.n = 3;
+    hs.v = 1;
     const int comp[3] = {DNSP_STEP_U, DNSP_STEP_V, DNSP_STEP_W};
-    const bool columns = s->d_bot[0] || s->d_bot[1] || s->d_bot[2];
-    const bool forcing = s->ibm[0] || s->ibm[1] || s->ibm[2];
-    if (columns) {
-        // each component's own columns; kmax = ny-1 for U, W and ny for V
-        // (mod_cfd_ibm.f90:47-141)
-        for (int c = 0; c < 3 && !rc; ++c)
-            if (s->d_bot[c])
-                rc = dnsp_ibm_part2(F[comp[c]], s->d_bot[c], s->d_top[c], nx, nz, ny, c == 1 ? ny : ny - 1,
-                                    s->walls[c], s->walls[3 + c], vs);
-        // cfd_periodicity (:860-899): halos, then U, W at k = -1, V at k = -1
-        // and 0, and all three at k = ny take the wall values
-        for (int c = 0; c < 3 && !rc; ++c) rc = dnsp_halo_periodic_xz(F[comp[c]], nx, nz, ny, vs);
-        for (int c = 0; c < 3 && !rc; ++c) {
-            rc = dnsp_set_val_slice(F[comp[c]], nx, nz, ny, 0, c == 1 ? 1 : 0, s->walls[c], vs);
-            if (!rc) rc = dnsp_set_val_slice(F[comp[c]], nx, nz, ny, -1, -1, s->walls[3 + c], vs);
-        }
-        if (rc) return rc;
+    for (int c = 0; c < 3; ++c) {
+        hs.A[c] = F[comp[c]];
+        hs.wb[c] = s->walls[c];
+        hs.wt[c] = s->walls[3 + c];
+        hs.bot[c] = s->d_bot[c];
+        hs.top[c] = s->d_top[c];
     }
-    if (forcing) {
-        for (int c = 0; c < 3 && !rc; ++c)
-            if (s->ibm[c]) rc = dnsp_ibm_exec(s->ibm[c], F[comp[c]], vs);
-        // ibm_part_1's wall planes: k = -1 and k = ny of U, V, W
-        for (int c = 0; c < 3 && !rc; ++c) {
-            rc = dnsp_set_val_slice(F[comp[c]], nx, nz, ny, 0, 0, s->walls[c], vs);
-            if (!rc) rc = dnsp_set_val_slice(F[comp[c]], nx, nz, ny, -1, -1, s->walls[3 + c], vs);
-        }
-    }
+    rc = halo_columns_periodicity(hs, nx, nz, ny, st);
+    if (!rc && (s->ibm[0] || s->ibm[1] || s->ibm[2])) rc = ibm_force_walls(s->ibm, hs, nx, nz, ny, st);
     return rc;
 }
 
