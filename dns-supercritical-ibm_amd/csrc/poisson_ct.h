@@ -1037,7 +1037,9 @@ __device__ __forceinline__ long tri_group_mode_mm(long grp, long ngroups, int mi
 // Grid: tri_groups(plane, M) workgroups of M * P threads, 3 * MR * P values
 // of type Ar of dynamic LDS.  With glist, workgroup b solves group
 // glist[b] (gridDim.x entries): the mixed form launches its FP32-arithmetic
-// groups and its FP64 ones from two such lists.
+// groups and its FP64 ones from two such lists.  A workgroup of 32 modes takes
+// two listed groups of 16 (-1: none), so that the lists split the modes 16 by 16
+// while neighbouring groups still make 128-byte FP32 rows.
 template <int MR, int P, int M, typename T = double, int OCC = 1, bool TP = false, typename Ar = double,
           bool MM = false>
 __global__ __launch_bounds__(M * P, OCC) void kt_tri_part(T* S, const double* __restrict__ ax,
@@ -1056,10 +1058,17 @@ __global__ __launch_bounds__(M * P, OCC) void kt_tri_part(T* S, const double* __
     // adjacent mode groups share cache lines: keep them on one XCD (each has
     // its own L2; workgroups reach XCDs round-robin)
     const int slot = xcd_tile((int)blockIdx.x, (int)gridDim.x);
-    const long grp = glist ? (long)glist[slot] : (long)slot;
+    long grp = glist ? (long)glist[slot] : (long)slot;
     long mode;
     if constexpr (MM) mode = tri_group_mode_mm<M>(grp, plane / M, mi, nx, nz);
     else mode = tri_group_mode(grp, (plane + M - 1) / M, M, mi);
+    if constexpr (M == 32) {
+        if (glist) {  // uniform
+            const int g16 = glist[2 * slot + mi / 16];
+            grp = glist[2 * slot];
+            mode = g16 < 0 ? LONG_MAX : tri_group_mode(g16, (plane + 15) / 16, 16, mi % 16);
+        }
+    }
     Ar d[MR];
     const double lam64 = tri_prologue<MR, P, M, T, Ar, MM>(d, smb, bands + (grp == 0 ? 3 * ny : 0), S, ax, az, mode,
                                                            plane, nx, ny, msum, nz);

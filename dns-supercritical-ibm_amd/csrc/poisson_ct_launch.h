@@ -69,38 +69,47 @@ int part_rows_for(int ny);  // rows per chunk at kPartChunks chunks (0: ny too l
 //   ny 384  P 16: 201 (0.94)  P 32: 203              before 247
 //   ny 770  P 32, M 8: 455 (0.83)  M 16: 555  P 16: 959  before 1403
 // Above 512 rows two workgroups of 16 modes no longer fit a CU's registers, so
-// a workgroup holds 8.
+// a workgroup holds 8.  FP32 spectra take twice the modes: 32 make 128-byte rows.
 struct PartShape {
     int P, M, MR;
 };
-constexpr PartShape part_shape(int ny) {
+constexpr PartShape part_shape(int ny, bool fp32 = false) {
     const int P = ny <= 48 ? 4 : (ny <= 128 ? 8 : (ny <= 512 ? 16 : 32));
     const int mr = (ny + P - 1) / P;
-    return {P, P == 32 ? 8 : 16, mr < 2 ? 2 : mr};
+    return {P, (P == 32 ? 8 : 16) * (fp32 ? 2 : 1), mr < 2 ? 2 : mr};
 }
-// The variant a handle starts with: part_shape's, two-pass from 21 rows a chunk
-// (at 24 rows 201 against 206 us, at 25 455 against 477; at 18 one-pass 146
-// against 149).
-constexpr int part_default_variant(int ny) { return part_shape(ny).MR > 20 ? 6 : 2; }
-// modes per workgroup (M) of a tridiagonal variant, FP32 or FP64 spectra
-int part_group_modes(int variant, int ny, bool fp32);
+// The variant a handle starts with, FP32 or FP64 spectra: part_shape's,
+// one-pass.  Two passes save registers but solve a chunk's interior again;
+// measured (us, one- against two-pass; mode-major and in place): 384x192x336
+// 84/86 and 65/72, 384x192x512 131/136 and 152/153, 576x288x400 220/242 and
+// 244/249, 624x312x770 657/722 and 679/752, 96x48x1000 33/35 and 32/36.
+constexpr int kPartDefault = 2;
+// The group lists of an FP32-spectrum variant (the mixed form launches the
+// well-conditioned groups in FP32 arithmetic and the rest in FP64): 0 = groups
+// of 8 modes, 1 = of 16, 2 and 3 = 32-mode workgroups whose lists hold pairs of
+// 16-mode groups, paired where all 32 modes qualify (2) or 16 by 16 (3).
+enum PartList { PL_8 = 0, PL_16 = 1, PL_32 = 2, PL_PAIRS = 3 };
+int part_list_kind(int variant, int ny);
 // Ar: arithmetic type (double, or float for FP32 spectra); glist (device,
 // nlist entries): solve only the listed mode groups (NULL: all of them);
 // MM: S in the mode-major blocks of the blocked solve, the solution written
 // to So in its x-blocked layout.
-// The arguments of a rule-shaped FP64 launch (poisson_tri_rule_*.hip).
+// The arguments of a rule-shaped launch (poisson_tri_rule_*.hip).
+template <typename T>
 struct PartArgs {
-    double* S;
+    T* S;
     const double *ax, *az, *bands;
     int nx, nz, ny;
     double pcr_min;
     const double* msum;
     double* pbar;
     double inv_nxnz;
-    double* So;
+    const int* glist;
+    int nlist;
+    T* So;
 };
-template <bool TP, bool MM>
-void part_launch_rule(const PartArgs& a, hipStream_t st);
+template <typename T, typename Ar, bool TP, bool MM>
+void part_launch_rule(const PartArgs<T>& a, hipStream_t st);
 template <typename T, typename Ar = double, bool MM = false>
 void part_launch(int variant, T* S, const double* ax, const double* az, const double* bands, int nx, int nz,
                  int ny, double pcr_min, const double* msum, double* pbar, double inv_nxnz, hipStream_t st,

@@ -38,8 +38,8 @@ struct dnsp_poisson {
     double* d_W = nullptr;            // its workspace, nx*nz*ny doubles
     int bxvar = 0, bxvar_b = 2;       // its x variants (forward, inverse)
     int bzvar = 1, bzvar_b = 1;       // its z variants (0: 256, 1: 512 threads)
-    int btvar = 4;                    // its tridiagonal variant
-    int tvar = 1;                     // partitioned tridiagonal variant
+    int btvar = 2;                    // its tridiagonal variant
+    int tvar = 2;                     // partitioned tridiagonal variant
     int part_rows = 0;                // partitioned tridiagonal rows per chunk (0 = serial)
     double* d_host = nullptr;  // staging for dnsp_poisson_run_host
     double min_pivot = 0;
@@ -60,11 +60,11 @@ struct dnsp_poisson {
     double* d_lsB = nullptr;
     double* d_small = nullptr;  // msum, pbar0, pbar1, q (ny each), residual partials
     double* d_fcopy = nullptr;  // copy of an in-place right-hand side (allocated when used)
-    // mode groups of the mixed tridiagonal for M = 8, 16, 32 modes per group:
-    // list [m][0] (FP64 arithmetic: a mode with |lambda| < f32_min, mode 0
-    // and the group of modes 1..M-1) and [m][1] (FP32 arithmetic), in d_glist
+    // mode groups of the mixed tridiagonal per list kind (part_list_kind):
+    // list [kind][0] (FP64 arithmetic: a mode with |lambda| < f32_min, mode 0
+    // and the group of modes 1..M-1) and [kind][1] (FP32 arithmetic), in d_glist
     int* d_glist = nullptr;
-    int gl_off[3][2] = {}, gl_n[3][2] = {};
+    int gl_off[4][2] = {}, gl_n[4][2] = {};
     size_t gl_total = 0;    // ints in d_glist
     double f32_min = 0;     // |lambda| from which a mode's sweeps run in FP32
     bool f32_sweeps = true; // FP32 arithmetic for the well-conditioned groups

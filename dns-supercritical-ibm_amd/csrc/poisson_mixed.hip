@@ -172,26 +172,36 @@ static int make_group_lists(dnsp_poisson* h) {
     h->f32_min = cmax / kF32Cond;
     const long plane = (long)nx * nz;
     std::vector<int> all;
-    const int Ms[3] = {8, 16, 32};
-    for (int mi = 0; mi < 3; ++mi) {
-        const int M = Ms[mi];
+    std::vector<char> ok((size_t)((plane + 7) / 8), 1);  // 8 modes at a time
+    for (int b = 0; b < nz; ++b)
+        for (int a = 0; a < nx; ++a)
+            if (!(std::fabs(ax[(size_t)a] + az[(size_t)b]) >= h->f32_min)) ok[(size_t)(((long)b * nx + a) / 8)] = 0;
+    auto well = [&](long m0, long n) {  // the modes m0..m0+n-1 of the plane, multiples of 8
+        for (long g = m0 / 8; g < std::min((long)ok.size(), (m0 + n) / 8); ++g)
+            if (!ok[(size_t)g]) return false;
+        return true;
+    };
+    for (int kind : {PL_8, PL_16, PL_32, PL_PAIRS}) {
+        const int M = kind == PL_8 ? 8 : 16;   // modes per listed group
+        const int W = kind == PL_32 ? 32 : M;  // modes that take one list together
         const long ngroups = (plane + M - 1) / M;
         std::vector<int> lo, hi;
+        hi.reserve((size_t)ngroups + 2);
         lo.push_back(0);
-        lo.push_back((int)ngroups);  // modes 1..M-1
+        if (kind >= PL_32) lo.push_back(-1);  // mode 0's workgroup stages its own bands
+        lo.push_back((int)ngroups);           // modes 1..M-1
         for (long g = 1; g < ngroups; ++g) {
-            bool f32 = true;
-            for (long m = g * M; m < std::min(plane, (g + 1) * M) && f32; ++m) {
-                const double lam = ax[(size_t)(m % nx)] + az[(size_t)(m / nx)];
-                f32 = std::fabs(lam) >= h->f32_min;
-            }
-            (f32 ? hi : lo).push_back((int)g);
+            const long m0 = g * M / W * W;
+            (m0 > 0 && well(m0, W) ? hi : lo).push_back((int)g);
         }
-        h->gl_off[mi][0] = (int)all.size();
-        h->gl_n[mi][0] = (int)lo.size();
+        if (kind >= PL_32)
+            for (std::vector<int>* l : {&lo, &hi})
+                if (l->size() % 2) l->push_back(-1);
+        h->gl_off[kind][0] = (int)all.size();
+        h->gl_n[kind][0] = (int)lo.size();
         all.insert(all.end(), lo.begin(), lo.end());
-        h->gl_off[mi][1] = (int)all.size();
-        h->gl_n[mi][1] = (int)hi.size();
+        h->gl_off[kind][1] = (int)all.size();
+        h->gl_n[kind][1] = (int)hi.size();
         all.insert(all.end(), hi.begin(), hi.end());
     }
     h->gl_total = all.size();
@@ -222,7 +232,15 @@ int mixed_setup(dnsp_poisson* h) {
     if (rc) return rc;
     DNSP_HIP_TRY(hipMalloc(&h->d_A, sizeof(float) * N));
     DNSP_HIP_TRY(hipMalloc(&h->d_B, sizeof(float) * N));
-    h->mtvar = 0;
+    // us per solve with one refinement.  Tridiagonal: the shape by ny against
+    // the (32, 16) shape that ran before: 64x32x64 59 / 71, 256x128x192 179 / 196,
+    // 512x256x256 725 / 745, 512x512x288 1757 / 1843.  z: 512 threads above 128
+    // points (128x192x128 131 / 135), with the 6144-element tile where the
+    // 3072-element one leaves rows of 96 bytes and the tiles stay many
+    // (193..256 points: 256x256x96 176 / 181, 512x256x256 698 / 725; at 384:
+    // 192x384x96 209 / 195).
+    h->mtvar = kPartDefault;
+    h->mzvar = h->nz <= 128 ? 0 : (h->nz > 192 && h->nz <= 256 ? 3 : 1);
     return make_group_lists(h);
 }
 
@@ -293,8 +311,7 @@ void mixed_tri(const dnsp_poisson* h, int variant, float* S, const double* msum,
                                    pbar, inv, st);
         return;
     }
-    const int M = part_group_modes(variant, h->ny, true);
-    const int mi = M == 8 ? 0 : (M == 16 ? 1 : 2);
+    const int mi = part_list_kind(variant, h->ny);
     part_launch<float, double>(variant, S, h->d_ax, h->d_az, h->d_bands, h->nx, h->nz, h->ny, h->pcr_min, msum, pbar,
                                inv, st, h->d_glist + h->gl_off[mi][0], h->gl_n[mi][0]);
     part_launch<float, float>(variant, S, h->d_ax, h->d_az, h->d_bands, h->nx, h->nz, h->ny, h->pcr_min, msum, pbar,
@@ -700,8 +717,8 @@ int dnsp_poisson_mixed_info(const dnsp_poisson* h, int* fp32_on, double* f32_min
     if (f32_min) *f32_min = h->f32_min;
     if (fp32_modes) {
         // modes of the FP32 groups of the variant in use
-        const int M = part_group_modes(h->mtvar, h->ny, true);
-        const int mi = M == 8 ? 0 : (M == 16 ? 1 : 2);
+        const int mi = part_list_kind(h->mtvar, h->ny);
+        const int M = mi == PL_8 ? 8 : 16;
         const long plane = (long)h->nx * h->nz;
         long long n = 0;
         if (h->f32_sweeps) {
@@ -709,7 +726,8 @@ int dnsp_poisson_mixed_info(const dnsp_poisson* h, int* fp32_on, double* f32_min
             if (!g.empty())
                 DNSP_HIP_TRY(hipMemcpy(g.data(), h->d_glist + h->gl_off[mi][1], sizeof(int) * g.size(),
                                        hipMemcpyDeviceToHost));
-            for (int q : g) n += std::min<long>(M, plane - (long)q * M);
+            for (int q : g)
+                if (q >= 0) n += std::min<long>(M, plane - (long)q * M);
         }
         *fp32_modes = n;
     }

@@ -17,11 +17,12 @@ static int rows_for(int ny, int chunks) {
 
 int part_rows_for(int ny) { return rows_for(ny, kPartChunks); }
 
-int part_group_modes(int variant, int ny, bool fp32) {
+int part_list_kind(int variant, int ny) {
     switch (variant) {
-        case 1: case 5: return 8;
-        case 3: case 7: return fp32 ? (ny <= 16 * 32 ? 32 : 16) : (ny <= 16 * 32 ? 16 : 8);
-        default: return 16;
+        case 1: case 5: return PL_8;
+        case 2: case 6: return part_shape(ny, true).M == 32 ? PL_PAIRS : PL_16;
+        case 3: case 7: return ny <= 16 * 32 ? PL_32 : PL_16;
+        default: return PL_16;
     }
 }
 
@@ -31,7 +32,7 @@ static void part_launch_mr(T* S, const double* ax, const double* az, const doubl
                            const int* glist, int nlist, T* So) {
     const long plane = (long)nx * nz;
     // every group, plus the group of modes 1..M-1; or the listed ones
-    const int ngroups = glist ? nlist : (int)((plane + M - 1) / M) + 1;
+    const int ngroups = glist ? nlist / (M == 32 ? 2 : 1) : (int)((plane + M - 1) / M) + 1;
     if (ngroups <= 0) return;
     const size_t lds = 3 * sizeof(Ar) * MR * P;
     kt_tri_part<MR, P, M, T, OCC, TP, Ar, MM><<<ngroups, M * P, lds, st>>>(S, ax, az, bands, nx, ny, plane, pcr_min,
@@ -62,6 +63,12 @@ void part_launch(int variant, T* S, const double* ax, const double* az, const do
 #define DNSP_PV(P, M, OCC, TP)                                                                                    \
     part_launch_pm<P, M, T, OCC, TP, Ar, MM>(S, ax, az, bands, nx, nz, ny, pcr_min, msum, pbar, inv_nxnz, st, glist, \
                                              nlist, So)
+    if (variant == 2 || variant == 6) {
+        const PartArgs<T> a{S, ax, az, bands, nx, nz, ny, pcr_min, msum, pbar, inv_nxnz, glist, nlist, So};
+        if (variant == 2) part_launch_rule<T, Ar, false, MM>(a, st);
+        else part_launch_rule<T, Ar, true, MM>(a, st);
+        return;
+    }
     if constexpr (sizeof(T) == 4) {
         // FP32 spectra: (16, 32) in place of (64, 8), whose 8-mode FP32 rows
         // are 32-byte segments (32 modes make a 128-byte row).  16 chunks of
@@ -71,14 +78,12 @@ void part_launch(int variant, T* S, const double* ax, const double* az, const do
         switch (variant) {
             case 0: DNSP_PV(32, 16, 4, false); break;
             case 1: DNSP_PV(32, 8, 1, false); break;
-            case 2: DNSP_PV(48, 16, 1, false); break;
             case 3:
                 if (c16) DNSP_PV(16, 32, 1, false);
                 else DNSP_PV(32, 16, 4, false);
                 break;
             case 4: DNSP_PV(32, 16, 4, true); break;
             case 5: DNSP_PV(32, 8, 1, true); break;
-            case 6: DNSP_PV(48, 16, 1, true); break;
             default:
                 if (c16) DNSP_PV(16, 32, 1, true);
                 else DNSP_PV(32, 16, 4, true);
@@ -89,14 +94,6 @@ void part_launch(int variant, T* S, const double* ax, const double* az, const do
     // FP64: 3 and 7 are (16, 16) for ny <= 512 (16 chunks of twice the
     // rows, one reduction step fewer), else (64, 8)
     const bool c16 = ny <= 16 * 32;
-    if constexpr (sizeof(T) == 8) {
-        if (variant == 2 || variant == 6) {
-            const PartArgs a{S, ax, az, bands, nx, nz, ny, pcr_min, msum, pbar, inv_nxnz, So};
-            if (variant == 2) part_launch_rule<false, MM>(a, st);
-            else part_launch_rule<true, MM>(a, st);
-            return;
-        }
-    }
     switch (variant) {
         case 0: DNSP_PV(32, 16, 4, false); break;
         case 1: DNSP_PV(32, 8, 1, false); break;

@@ -1,0 +1,6 @@
+// One-pass rule-shaped tridiagonal kernels, FP32 spectra and arithmetic.
+#define DNSP_RULE_T float
+#define DNSP_RULE_AR float
+#define DNSP_RULE_TP false
+#define DNSP_RULE_MM false
+#include "poisson_tri_rule.h"

@@ -182,10 +182,10 @@ int dnsp_poisson_get_strategy(const dnsp_poisson* h, int* fft_ct_x, int* fft_ct_
  * (2), (16, 16) for ny <= 512, else (64, 8) (3); rows per chunk follow from ny.
  * 4..7: the same shapes with two-pass chunks (the chunk interior is solved
  * again once its end values are known, instead of being kept in registers
- * across the reduced solve).  A handle starts with 2, or 6 where a chunk has
- * more than 20 rows.  The mixed-precision form has its own set; on its FP32
- * spectra shapes 2 and 6 are (48, 16), 3 and 7 (16, 32), whose 32 modes make
- * 128-byte rows.  No counterpart in the reference. */
+ * across the reduced solve).  A handle starts with 2.  The mixed-precision
+ * form has its own set; on its FP32 spectra shapes 2 and 6 have twice the modes
+ * (32, and 16 above 512 rows), 3 and 7 are (16, 32): 32 modes make 128-byte
+ * rows.  No counterpart in the reference. */
 int dnsp_poisson_set_variants(dnsp_poisson* h, int xvar, int zvar, int tvar);
 int dnsp_poisson_get_variants(const dnsp_poisson* h, int* xvar, int* zvar, int* tvar);
 int dnsp_poisson_set_mixed_variants(dnsp_poisson* h, int xvar, int zvar, int tvar);

@@ -63,3 +63,30 @@ def test_rule_shapes_match_serial_and_blocked(cuda, ny):
             out.append(to_host(P))
         assert np.abs(out[1] - out[0]).max() <= 1e-13 * np.abs(out[0]).max(), tv
     s.close()
+
+
+@pytest.mark.parametrize("ny", [2, 8, 33, 48, 49, 96, 128, 129, 280, 512, 513, 1024])
+def test_rule_shapes_of_fp32_spectra(cuda, ny):
+    """The mixed form's 32-mode shapes, whose two group lists pair 16-mode
+    groups: the same modes run in FP32 as with 16-mode workgroups, and one
+    refinement meets the residual bar of the other shapes (1e-10)."""
+    nx, nz = 96, 32
+    say("fp32 rule shape", ny)
+    yu = W.tanh_faces(ny, 1.2)
+    rhs = W.rhs_band_limited((ny, nz, nx), 2, yu=yu)
+    idx, idz = nx / W.LX, nz / W.LZ
+    bands = D.mk_P_abc(yu, False) + D.mk_P_abc(yu, True)
+    s = D.PoissonSolver(nx, nz, ny, idx, idz, bands, precision=D.PRECISION_MIXED)
+    src = to_dev(rhs)
+    s.set_mixed_variants(0, 0, 0)
+    n32 = s.mixed_info[2]
+    for tv in (2, 6):
+        s.set_mixed_variants(0, 0, tv)
+        assert s.mixed_info[2] == n32, tv
+        for fp32 in (False, True):
+            s.set_mixed_fp32(fp32)
+            P = to_dev(np.zeros_like(rhs))
+            s.solve_mixed(src, P, 1)
+            rel = s.residual(src, P)
+            assert rel <= 1e-10, (tv, fp32, rel)
+    s.close()
