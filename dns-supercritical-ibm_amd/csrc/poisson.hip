@@ -689,13 +689,8 @@ int dnsp_poisson_init(int nx_glob, int nz_glob, int ny, double inv_dx, double in
     h->inv_dz = inv_dz;
     h->precision = precision;
     h->tvar = h->btvar = kPartDefault;
-    // The blocked solve's x tiles (us).  Forward: 1536 complex elements a
-    // workgroup where the field outgrows the 256 MB cache (768x384x384 354
-    // against 368 for 768, 256x256x256 43 against 46), else 768 (512x128x192 35
-    // against 39).  Inverse: 768 at 384 and 512 points (384x384x256 100 against
-    // 105), else 1536 (256x256x256 39 against 41, 768x384x384 316 against 321).
-    h->bxvar = (size_t)nx_glob * (size_t)nz_glob * (size_t)ny >= ((size_t)1 << 24) ? 2 : 0;
-    h->bxvar_b = nx_glob == 384 || nx_glob == 512 ? 0 : 2;
+    h->bxvar = blk_xfwd_variant((size_t)nx_glob * (size_t)nz_glob * (size_t)ny);
+    h->bxvar_b = blk_xbwd_variant(nx_glob);
     int rc = poisson_setup(h, bands);
     if (!rc) rc = poisson_apply_strategy(h);
     if (!rc) rc = mixed_setup(h);

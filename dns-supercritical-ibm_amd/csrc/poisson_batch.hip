@@ -1,8 +1,9 @@
 // Batched Poisson solves of many independent instances of uneven sizes.
 //
-// Every stage of the solve is one launch per distinct transform length (x, z)
-// or rows-per-chunk (tridiagonal) covering the tiles of all instances of that
-// size: a workgroup decodes its task through a slot table (instance, tile)
+// Large instances of the FP64 form run one after the other through the blocked
+// single solve.  For the others every stage of the solve is one launch per
+// distinct transform length (x, z) or rows-per-chunk (tridiagonal) covering the
+// tiles of all instances of that size: a workgroup decodes its task through a slot table (instance, tile)
 // and runs the same tile bodies as the single-instance kernels.  A batch of
 // 48 instances over 5 x lengths, 5 z lengths and 4 row counts thus takes 24
 // launches per FP64 solve instead of 240.  The FP64 form and the
@@ -154,7 +155,20 @@ __global__ __launch_bounds__(ct_zvar_threads(V)) void kb_z(const BInst* __restri
 // (8 chunks of four times the rows measured the same as 16 on the
 // 48-instance batch: not kept.)
 constexpr int kBatchM = 8;
-constexpr int kBatchTriVariants = 6;
+// Points from which an instance runs alone.  By itself its stages stay in the
+// 256 MB cache and use the blocked layouts and full-width tridiagonal groups, but
+// five launches of its own leave gaps that a small one does not fill.  us per
+// million points, alone against shared (16 instances of one size): 192x96x130
+// 24.4 / 16.5, 256x96x192 (4.7 M) 18.5 / 15.8, 256x192x192 (9.4 M) 14.9 / 15.7,
+// 512x192x192 14.8 / 16.3.  Uneven batches whose sizes share few launches cross
+// earlier; 16 and 13 instances of 0.8..25 M points, ms by threshold: 2 M 2.50,
+// 1.18; 4.5 M 2.48, 1.13; 6 M 2.47, 1.11; 8 M 2.45, 1.13; none 2.73, 1.22.
+constexpr size_t kBatchAlone = (size_t)6 << 20;
+// 6 (FP64): an instance of at least kBatchAlone points runs by itself through
+// the blocked stages of the single solve (shape by ny with exact rows), the
+// instances share one workspace, and the smaller ones run as variant 4.
+constexpr int kBatchTriVariants = 7;
+constexpr int kBatchMixedTriVariants = 6;
 
 template <int MR, int KIND, int OCC, bool TP, int P = kPartChunks>
 __global__ __launch_bounds__(kBatchM * P, OCC) void kb_tri(const BInst* __restrict__ inst,
@@ -530,7 +544,13 @@ struct dnsp_batch {
     std::vector<BGroup> gx[kCtVariants], gz[kCtVariants], gt;
     BGroup gq;
     int max_ny = 0;
-    int xvar = 0, zvar = 0, tvar = 1;     // FP64 form
+    // variant 6: the instances that run alone and their workspace (NULL: none,
+    // or no memory for it, and every instance runs in the shared launches);
+    // the launch groups of the others
+    std::vector<int> alone;
+    double* d_W = nullptr;
+    std::vector<BGroup> sx[kCtVariants], sz[kCtVariants], st;
+    int xvar = 0, zvar = 1, tvar = 6;     // FP64 form
     int mxvar = 0, mzvar = 0, mtvar = 1;  // mixed form
     bool bound = false;
     // persistent launch (built at its first use): group table, plan, LDS
@@ -595,10 +615,11 @@ int twiddles(dnsp_batch* b, int n, V** out) {
     return dev_copy(b, out, tw.data(), (size_t)n);
 }
 
-// Groups instances by key; per instance `tasks` work items.
+// Groups instances by key; per instance `tasks` work items (0: not in a group).
 int make_groups(dnsp_batch* b, const std::vector<int>& key, const std::vector<long>& tasks, std::vector<BGroup>& out) {
     std::map<int, std::vector<int>> by;
-    for (int i = 0; i < b->n; ++i) by[key[(size_t)i]].push_back(i);
+    for (int i = 0; i < b->n; ++i)
+        if (tasks[(size_t)i] > 0) by[key[(size_t)i]].push_back(i);
     out.clear();
     for (auto& kv : by) {
         BGroup g;
@@ -622,10 +643,18 @@ int make_groups(dnsp_batch* b, const std::vector<int>& key, const std::vector<lo
             const long end = u + 1 < g.cnt ? st[(size_t)u + 1] : tot;
             for (long t = st[(size_t)u]; t < end; ++t) sl[(size_t)t] = u;
         }
-        int rc = dev_copy(b, &g.ids, kv.second.data(), kv.second.size());
-        if (!rc) rc = dev_copy(b, &g.start, st.data(), st.size());
-        if (!rc && tot > 0) rc = dev_copy(b, &g.slot, sl.data(), sl.size());
+        // one allocation and copy: start | ids | slot
+        const size_t cnt = st.size(), bytes = sizeof(long) * cnt + sizeof(int) * (cnt + sl.size());
+        std::vector<char> blob(bytes);
+        std::memcpy(blob.data(), st.data(), sizeof(long) * cnt);
+        std::memcpy(blob.data() + sizeof(long) * cnt, kv.second.data(), sizeof(int) * cnt);
+        std::memcpy(blob.data() + (sizeof(long) + sizeof(int)) * cnt, sl.data(), sizeof(int) * sl.size());
+        char* d = nullptr;
+        int rc = dev_copy(b, &d, blob.data(), bytes);
         if (rc) return rc;
+        g.start = reinterpret_cast<long*>(d);
+        g.ids = reinterpret_cast<int*>(d + sizeof(long) * cnt);
+        g.slot = g.ids + cnt;
         out.push_back(g);
     }
     return DNSP_OK;
@@ -722,8 +751,37 @@ int setup_eig(dnsp_batch* b, const double* inv_dx, const double* inv_dz) {
     return DNSP_OK;
 }
 
+// The instances variant 6 runs alone, and their workspace.
+int setup_alone(dnsp_batch* b) {
+    size_t most = 0;
+    for (int i = 0; i < b->n; ++i) {
+        const BInst& I = b->h_inst[(size_t)i];
+        const size_t N = (size_t)I.plane * (size_t)I.ny;
+        if (N < kBatchAlone) continue;
+        b->alone.push_back(i);
+        most = std::max(most, N);
+    }
+    if (!most) return DNSP_OK;
+    void* w = nullptr;
+    if (hipMalloc(&w, sizeof(double) * most) != hipSuccess) {  // the shared launches need none
+        (void)hipGetLastError();
+        b->alone.clear();
+        return DNSP_OK;
+    }
+    b->allocs.push_back(w);
+    b->d_W = static_cast<double*>(w);
+    return DNSP_OK;
+}
+
 int setup_groups(dnsp_batch* b) {
     const int n = b->n;
+    std::vector<char> shared((size_t)n, 1);
+    for (int i : b->alone) shared[(size_t)i] = 0;
+    auto rest = [&](std::vector<long> t) {  // the tasks of the instances that do not run alone
+        for (int i = 0; i < n; ++i)
+            if (!shared[(size_t)i]) t[(size_t)i] = 0;
+        return t;
+    };
     for (int v = 0; v < kCtVariants; ++v) {
         std::vector<long> tx((size_t)n), tz((size_t)n);
         for (int i = 0; i < n; ++i) {
@@ -736,6 +794,8 @@ int setup_groups(dnsp_batch* b) {
         }
         int rc = make_groups(b, b->nx, tx, b->gx[v]);
         if (!rc) rc = make_groups(b, b->nz, tz, b->gz[v]);
+        if (!rc && !b->alone.empty()) rc = make_groups(b, b->nx, rest(tx), b->sx[v]);
+        if (!rc && !b->alone.empty()) rc = make_groups(b, b->nz, rest(tz), b->sz[v]);
         if (rc) return rc;
     }
     std::vector<long> tt((size_t)n), tq((size_t)n);
@@ -746,6 +806,7 @@ int setup_groups(dnsp_batch* b) {
         tq[(size_t)i] = I.ny;
     }
     int rc = make_groups(b, b->mr, tt, b->gt);
+    if (!rc && !b->alone.empty()) rc = make_groups(b, b->mr, rest(tt), b->st);
     if (rc) return rc;
     if (b->precision == DNSP_PRECISION_MIXED) {
         // per row-count launch group: (slot, mode group) pairs with a mode of
@@ -795,13 +856,29 @@ int upload_inst(dnsp_batch* b) {
     return DNSP_OK;
 }
 
+// One instance through the blocked stages (dnsp_poisson_solve_stage).
+void run_alone(const BInst& I, double* W, hipStream_t st) {
+    const size_t N = (size_t)I.plane * (size_t)I.ny;
+    xb_x_launch(I.nx, blk_xfwd_variant(N), I.f, W, I.nlines, I.nz, I.twx, st);
+    mm_z_launch(I.nz, kBlkZVariant, false, W, I.P, I.nx, I.ny, I.twz, st);
+    part_launch<double, double, true>(kPartDefault, I.P, I.ax, I.az, I.bands, I.nx, I.nz, I.ny, I.pcr_min, nullptr,
+                                      nullptr, 0.0, st, nullptr, 0, W);
+    mm_z_launch(I.nz, kBlkZVariant, true, W, I.P, I.nx, I.ny, I.twz, st);
+    ct_x_launch(I.nx, blk_xbwd_variant(I.nx), true, I.P, I.P, I.nlines, I.twx, I.inv_nxnz, st);
+}
 
 void run_fp64(dnsp_batch* b, int xv, int zv, int tv, hipStream_t st) {
-    for (const BGroup& g : b->gx[xv]) bx_launch(BX_F64_FWD, xv, b->d_inst, g, 0, st);
-    for (const BGroup& g : b->gz[zv]) bz_launch(BZ_F64_FWD, zv, b->d_inst, g, st);
-    for (const BGroup& g : b->gt) bt_launch(0, tv, b->d_inst, g, st);
-    for (const BGroup& g : b->gz[zv]) bz_launch(BZ_F64_BWD, zv, b->d_inst, g, st);
-    for (const BGroup& g : b->gx[xv]) bx_launch(BX_F64_BWD, xv, b->d_inst, g, 0, st);
+    const bool split = tv == 6 && !b->alone.empty();
+    if (tv == 6) tv = 4;
+    if (split)
+        for (int i : b->alone) run_alone(b->h_inst[(size_t)i], b->d_W, st);
+    const std::vector<BGroup>&gx = split ? b->sx[xv] : b->gx[xv], &gz = split ? b->sz[zv] : b->gz[zv],
+                            &gt = split ? b->st : b->gt;
+    for (const BGroup& g : gx) bx_launch(BX_F64_FWD, xv, b->d_inst, g, 0, st);
+    for (const BGroup& g : gz) bz_launch(BZ_F64_FWD, zv, b->d_inst, g, st);
+    for (const BGroup& g : gt) bt_launch(0, tv, b->d_inst, g, st);
+    for (const BGroup& g : gz) bz_launch(BZ_F64_BWD, zv, b->d_inst, g, st);
+    for (const BGroup& g : gx) bx_launch(BX_F64_BWD, xv, b->d_inst, g, 0, st);
 }
 
 void run_mixed(dnsp_batch* b, int refinements, int xv, int zv, int tv, hipStream_t st) {
@@ -911,6 +988,7 @@ int dnsp_batch_create(int n, const int* nx, const int* nz, const int* ny, const 
     for (int i = 0; i < n; ++i) b->mr[(size_t)i] = part_rows_for(ny[i]);
     int rc = setup(b, bands);
     if (!rc) rc = setup_eig(b, inv_dx, inv_dz);
+    if (!rc) rc = setup_alone(b);
     if (!rc) rc = setup_groups(b);
     if (!rc) rc = upload_inst(b);
     if (rc) {
@@ -980,7 +1058,8 @@ int dnsp_batch_set_variants(dnsp_batch* b, int xvar, int zvar, int tvar, int mxv
     clear_error();
     DNSP_ARG_CHECK(b, "NULL batch");
     for (int v : {xvar, zvar, mxvar, mzvar}) DNSP_ARG_CHECK(v >= 0 && v < kCtVariants, "FFT variant %d", v);
-    for (int v : {tvar, mtvar}) DNSP_ARG_CHECK(v >= 0 && v < kBatchTriVariants, "tridiagonal variant %d", v);
+    DNSP_ARG_CHECK(tvar >= 0 && tvar < kBatchTriVariants, "tridiagonal variant %d", tvar);
+    DNSP_ARG_CHECK(mtvar >= 0 && mtvar < kBatchMixedTriVariants, "mixed tridiagonal variant %d", mtvar);
     b->xvar = xvar;
     b->zvar = zvar;
     b->tvar = tvar;
@@ -1023,7 +1102,7 @@ int dnsp_batch_autotune(dnsp_batch* b, int reps, void* stream, double* times_ms)
         if (form == 1 && b->precision != DNSP_PRECISION_MIXED) break;
         int* var[3] = {form ? &b->mxvar : &b->xvar, form ? &b->mzvar : &b->zvar, form ? &b->mtvar : &b->tvar};
         for (int knob = 0; knob < 3 && rc == DNSP_OK; ++knob) {
-            const int nv = knob == 2 ? kBatchTriVariants : kCtVariants;
+            const int nv = knob < 2 ? kCtVariants : (form ? kBatchMixedTriVariants : kBatchTriVariants);
             double best = 1e30;
             int pick = *var[knob];
             for (int v = 0; v < nv; ++v) {

@@ -37,7 +37,7 @@ struct dnsp_poisson {
     bool blk_on = true;               // used by dnsp_poisson_run / solve when supported
     double* d_W = nullptr;            // its workspace, nx*nz*ny doubles
     int bxvar = 0, bxvar_b = 2;       // its x variants (forward, inverse)
-    int bzvar = 1, bzvar_b = 1;       // its z variants (0: 256, 1: 512 threads)
+    int bzvar = dnsp::kBlkZVariant, bzvar_b = dnsp::kBlkZVariant;       // its z variants (0: 256, 1: 512 threads)
     int btvar = 2;                    // its tridiagonal variant
     int tvar = 2;                     // partitioned tridiagonal variant
     int part_rows = 0;                // partitioned tridiagonal rows per chunk (0 = serial)

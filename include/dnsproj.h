@@ -250,7 +250,8 @@ int dnsp_poisson_mixed_info(const dnsp_poisson* h, int* fp32_on, double* f32_min
  * Batched form: many independent solves of uneven sizes (no counterpart in
  * the reference, which solves one field per rank).  Each stage of the solve
  * is one launch per distinct transform length (x, z) or rows-per-chunk
- * (tridiagonal) over the tiles of all instances of that size.
+ * (tridiagonal) over the tiles of all instances of that size; FP64 instances
+ * of 6 * 2^20 points and more run by themselves, one after the other.
  *   dnsp_batch_create: n instances; nx[i], nz[i] in {32,64,96,128,192,256,384,
  *     512,768}, 2 <= ny[i] <= 1024; bands = the instances' six band arrays
  *     (a, b, c, a00, b00, c00, ny[i] each) concatenated in instance order;
@@ -268,7 +269,11 @@ int dnsp_poisson_mixed_info(const dnsp_poisson* h, int* fp32_on, double* f32_min
  *     32 chunks, 1 = the same with registers capped for 4 waves per SIMD, 2
  *     and 3 = 0 and 1 with two-pass chunks, 4 and 5 = 8-mode groups of 16
  *     chunks of twice the rows, one-pass and two-pass (32 chunks where the
- *     rows would exceed 32)), keeps the fastest; overwrites the bound P
+ *     rows would exceed 32), 6 (FP64 only, the default) = 4, with the
+ *     instances of 6 * 2^20 points and more solved one by one as
+ *     dnsp_poisson_solve does, through one workspace of the largest's size
+ *     that create allocates (as 4 if it cannot); x and z variants then apply
+ *     to the smaller ones), keeps the fastest; overwrites the bound P
  *     arrays; times_ms as for dnsp_poisson_autotune.  Synchronises.
  *   dnsp_batch_set_variants / get_variants: FP64 x, z, tridiagonal, then the
  *     mixed form's (6 ints).
