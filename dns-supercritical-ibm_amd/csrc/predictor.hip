@@ -117,16 +117,14 @@ __global__ void k_div_finish(double* D, Grid g) {
 // buoyancy field (read at the point and at (-1, 0, 0), (0, -1, 0), (0, 0, -1)).
 template <bool VARPROP, class AU, class AV, class AW, class AM, class AR, class AD, class AB>
 __device__ __forceinline__ void momentum_point(
-    const AU& u, const AV& v, const AW& w, const AM& m, const AR& r, const AD& dv, const AB& b, int i, int j, int k,
-    double* __restrict__ Ru_old, double* __restrict__ Rv_old, double* __restrict__ Rw_old,
+    const AU& u, const AV& v, const AW& w, const AM& m, const AR& r, const AD& dv, const AB& b, long c, long o, int k, double ru_old,
+    double rv_old, double rw_old, double* __restrict__ Ru_old, double* __restrict__ Rv_old, double* __restrict__ Rw_old,
     double* __restrict__ U_hat, double* __restrict__ V_hat, double* __restrict__ W_hat, const Grid& g,
     const Geom& G, const Phys& p, int kmin_Vhat) {
-    const long c = g.at(i, j, k);
-    const long o = (long)i + (long)g.nx * ((long)j + (long)g.nz * k);
     const double idx = p.idx, idz = p.idz, idx2 = p.idx2, idz2 = p.idz2, idx__2 = p.idx__2, idz__2 = p.idz__2;
     {
-        const double Ra = G.ruw[3 * k], Rb = G.ruw[3 * k + 1], Rc = G.ruw[3 * k + 2];
-        const double R2a = G.ruw2[3 * k], R2b = G.ruw2[3 * k + 1], R2c = G.ruw2[3 * k + 2];
+        const double Ra = uniform_load(G.ruw, 3 * k), Rb = uniform_load(G.ruw, 3 * k + 1), Rc = uniform_load(G.ruw, 3 * k + 2);
+        const double R2a = uniform_load(G.ruw2, 3 * k), R2b = uniform_load(G.ruw2, 3 * k + 1), R2c = uniform_load(G.ruw2, 3 * k + 2);
         const double dudx = (u(1, 0, 0) - u(-1, 0, 0)) * idx__2;
         const double dudz = (u(0, 1, 0) - u(0, -1, 0)) * idz__2;
         const double dudy = (u(0, 0, -1) * Ra + u(0, 0, 0) * Rb) + u(0, 0, 1) * Rc;
@@ -183,17 +181,17 @@ __device__ __forceinline__ void momentum_point(
                      (0.5 * (r(0, -1, 0) + r(0, 0, 0)));
             }
         }
-        U_hat[c] = u(0, 0, 0) + p.dt * (1.5 * Ru - 0.5 * Ru_old[o]);
-        W_hat[c] = w(0, 0, 0) + p.dt * (1.5 * Rw - 0.5 * Rw_old[o]);
+        U_hat[c] = u(0, 0, 0) + p.dt * (1.5 * Ru - 0.5 * ru_old);
+        W_hat[c] = w(0, 0, 0) + p.dt * (1.5 * Rw - 0.5 * rw_old);
         Ru_old[o] = Ru;
         Rw_old[o] = Rw;
     }
     if (k < kmin_Vhat) return;
     {
-        const double Va = G.rv[3 * k], Vb = G.rv[3 * k + 1], Vc = G.rv[3 * k + 2];
-        const double V2a = G.rv2[3 * k], V2b = G.rv2[3 * k + 1], V2c = G.rv2[3 * k + 2];
-        const double ib = G.itp[2 * k], it = G.itp[2 * k + 1];
-        const double idyu = G.idyu[k];
+        const double Va = uniform_load(G.rv, 3 * k), Vb = uniform_load(G.rv, 3 * k + 1), Vc = uniform_load(G.rv, 3 * k + 2);
+        const double V2a = uniform_load(G.rv2, 3 * k), V2b = uniform_load(G.rv2, 3 * k + 1), V2c = uniform_load(G.rv2, 3 * k + 2);
+        const double ib = uniform_load(G.itp, 2 * k), it = uniform_load(G.itp, 2 * k + 1);
+        const double idyu = uniform_load(G.idyu, k);
         const double dvdx = (v(1, 0, 0) - v(-1, 0, 0)) * idx__2;
         const double dvdz = (v(0, 1, 0) - v(0, -1, 0)) * idz__2;
         const double dvdy = (v(0, 0, -1) * Va + v(0, 0, 0) * Vb) + v(0, 0, 1) * Vc;
@@ -219,7 +217,7 @@ __device__ __forceinline__ void momentum_point(
             const double visc = (((0.5 * (m(0, 0, -1) + m(0, 0, 0))) * D + E * Fx) + Gt * H) + I * J;
             Rv = ((-conv + visc) + p.Gb_y * (0.5 * (b(0, 0, 0) + b(0, 0, -1)))) / (0.5 * (r(0, 0, -1) + r(0, 0, 0)));
         }
-        V_hat[c] = v(0, 0, 0) + p.dt * (1.5 * Rv - 0.5 * Rv_old[o]);
+        V_hat[c] = v(0, 0, 0) + p.dt * (1.5 * Rv - 0.5 * rv_old);
         Rv_old[o] = Rv;
     }
 }
@@ -227,10 +225,17 @@ __device__ __forceinline__ void momentum_point(
 // U, V, W (and mu) are read at up to 16 neighbouring points each, so a
 // workgroup stages them in LDS (PlaneRing, stencil_grid.h): it owns a 64 x 4
 // (i, j) tile and marches through a run of planes with planes k-1, k, k+1 of
-// each field in a ring of three slots, the next plane's loads issued before
+// each field in a ring of slots, the next plane's loads issued before
 // a step's arithmetic.  rho, div_now and buoyancy (four points each) are
 // read directly.  The per-thread version made 12.5 L1 and 2.9 L2 read
 // requests per point.
+// A step consumes no vector load of its own: the other fields' values are loaded
+// a plane ahead and the coefficients are scalar loads, because loads return in
+// order and a wait for a late one waits for the whole prefetch (the version with
+// loads inside the step waited for everything outstanding five times a plane:
+// 683 us at 384x192x256, 3.9 TB/s over 93 + 48 B/pt from beyond L2; now 565 us,
+// 4.7 TB/s).  203 VGPRs, two waves per SIMD; capped for three: 577 us; two planes
+// of the ring in flight instead of one: 562, and 2% more on small grids.
 template <bool VARPROP>
 __global__ __launch_bounds__(kThreads) void k_momentum(
     const double* __restrict__ U, const double* __restrict__ V, const double* __restrict__ W,
@@ -239,59 +244,77 @@ __global__ __launch_bounds__(kThreads) void k_momentum(
     double* __restrict__ Rw_old, double* __restrict__ U_hat, double* __restrict__ V_hat, double* __restrict__ W_hat,
     Grid g, BandGrid bg, Geom G, Phys p, int kmin_Vhat) {
     constexpr int NF = VARPROP ? 4 : 3;
-    __shared__ double sF[NF][3][kRingP];
+    __shared__ double sF[NF][kRingSlots][kRingP];
     int i0, j0, k0, k1;
     if (!ring_tile(bg, g.ny, i0, j0, k0, k1)) return;
-    const int i = i0 + (int)threadIdx.x, j = j0 + (int)threadIdx.y;
-    const bool active = i < g.nx && j < g.nz;
     const double* fields[4] = {U, V, W, mu};
     PlaneRing<NF> ring(sF, fields, i0, j0, g.nx, g.nz);
     ring.prime(k0);
-    const int e0 = ring_point();
-    const long sz = g.sz(), sy = g.sy();
-    // rho, div_now and buoy of this thread's column at plane k - 1: read at
-    // the march's first plane, then carried from the step before (the plane
-    // below is otherwise read again from beyond L2 once the step's other
-    // streams have pushed it out)
-    double rm = 0.0, dm = 0.0, bm = 0.0;
-    if (VARPROP && active) {
-        const long cm = g.at(i, j, k0 - 1);
-        rm = rho[cm];
-        dm = dvn[cm];
-        bm = buoy[cm];
+    // lanes past the last column repeat its point (same loads, same stores)
+    const int row = tile_row(), j = j0 + row;
+    if (j >= g.nz) {
+        ring.stage(k0, k1);
+        return;
     }
-    for (int k = k0; k < k1; ++k) {
-        ring.put(k + 1);  // the slot of plane k - 2, free since the last barrier
-        __syncthreads();
-        if (k + 2 <= k1) ring.fetch(k + 2);  // in flight during this step's arithmetic
-        if (active) {
-            const int sm = (k + 2) % 3, s0 = k % 3, sp = (k + 1) % 3;
-            auto slot = [&](int dk) { return dk < 0 ? sm : (dk > 0 ? sp : s0); };
-            auto lu = [&](int di, int dj, int dk) { return sF[0][slot(dk)][e0 + di + dj * kRingX]; };
-            auto lv = [&](int di, int dj, int dk) { return sF[1][slot(dk)][e0 + di + dj * kRingX]; };
-            auto lw = [&](int di, int dj, int dk) { return sF[2][slot(dk)][e0 + di + dj * kRingX]; };
-            auto lm = [&](int di, int dj, int dk) { return sF[NF - 1][slot(dk)][e0 + di + dj * kRingX]; };
-            const long c = g.at(i, j, k);
-            double r0 = 0.0, d0 = 0.0, b0 = 0.0;
-            if constexpr (VARPROP) {
-                r0 = rho[c];
-                d0 = dvn[c];
-                b0 = buoy[c];
+    const int i = min(i0 + (int)threadIdx.x, g.nx - 1);
+    const int e0 = (row + 1) * kRingX + (i - i0) + 1;
+    const long sz = g.sz(), sy = g.sy();
+    // this point's rho, div_now and buoy with their x and z neighbours, and the
+    // last step's R: loaded a plane ahead
+    struct Ahead {
+        double cen[3], x[3], z[3], old[3];
+    };
+    auto ahead = [&](int k) {
+        Ahead a{};
+        const long c = g.at(i, j, k);
+        const long o = (long)i + (long)g.nx * ((long)j + (long)g.nz * k);
+        if constexpr (VARPROP) {
+            const double* f[3] = {rho, dvn, buoy};
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                a.cen[q] = f[q][c];
+                a.x[q] = f[q][c - 1];
+                a.z[q] = f[q][c - sz];
             }
-            // (0, 0, -1) from registers, (0, 0, 0) as loaded, x and z neighbours from memory
-            auto at = [&](const double* f, double cen, double below, int di, int dj, int dk) {
-                return dk < 0 ? below : ((di | dj) == 0 ? cen : f[c + di + dj * sz + dk * sy]);
-            };
-            auto lr = [&](int di, int dj, int dk) { return at(rho, r0, rm, di, dj, dk); };
-            auto ld = [&](int di, int dj, int dk) { return at(dvn, d0, dm, di, dj, dk); };
-            auto lb = [&](int di, int dj, int dk) { return at(buoy, b0, bm, di, dj, dk); };
-            momentum_point<VARPROP>(lu, lv, lw, lm, lr, ld, lb, i, j, k, Ru_old, Rv_old, Rw_old, U_hat, V_hat, W_hat,
-                                    g, G, p, kmin_Vhat);
-            rm = r0;
-            dm = d0;
-            bm = b0;
         }
-        __syncthreads();  // slot (k + 2) % 3 is restaged next
+        a.old[0] = Ru_old[o];
+        a.old[1] = Rv_old[o];
+        a.old[2] = Rw_old[o];
+        return a;
+    };
+    // rho, div_now and buoy at plane k - 1: carried from the step before
+    double below[3] = {};
+    if constexpr (VARPROP) {
+        const long cm = g.at(i, j, k0 - 1);
+        below[0] = rho[cm];
+        below[1] = dvn[cm];
+        below[2] = buoy[cm];
+    }
+    Ahead nx = ahead(k0);
+    for (int k = k0; k < k1; ++k) {
+        ring.put(k + 1);
+        const Ahead a = nx;
+        __syncthreads();
+        // in flight during this step's arithmetic
+        ring.fetch(min(k + 2, k1));
+        nx = ahead(min(k + 1, k1 - 1));
+        const int sm = ring_slot(k - 1), s0 = ring_slot(k), sp = ring_slot(k + 1);
+        auto slot = [&](int dk) { return dk < 0 ? sm : (dk > 0 ? sp : s0); };
+        auto lu = [&](int di, int dj, int dk) { return sF[0][slot(dk)][e0 + di + dj * kRingX]; };
+        auto lv = [&](int di, int dj, int dk) { return sF[1][slot(dk)][e0 + di + dj * kRingX]; };
+        auto lw = [&](int di, int dj, int dk) { return sF[2][slot(dk)][e0 + di + dj * kRingX]; };
+        auto lm = [&](int di, int dj, int dk) { return sF[NF - 1][slot(dk)][e0 + di + dj * kRingX]; };
+        auto at = [&](int q, int di, int dj, int dk) {
+            return dk < 0 ? below[q] : (di < 0 ? a.x[q] : (dj < 0 ? a.z[q] : a.cen[q]));
+        };
+        auto lr = [&](int di, int dj, int dk) { return at(0, di, dj, dk); };
+        auto ld = [&](int di, int dj, int dk) { return at(1, di, dj, dk); };
+        auto lb = [&](int di, int dj, int dk) { return at(2, di, dj, dk); };
+        momentum_point<VARPROP>(lu, lv, lw, lm, lr, ld, lb, g.at(i, j, k),
+                                (long)i + (long)g.nx * ((long)j + (long)g.nz * k), k, a.old[0], a.old[1], a.old[2],
+                                Ru_old, Rv_old, Rw_old, U_hat, V_hat, W_hat, g, G, p, kmin_Vhat);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) below[q] = a.cen[q];
     }
 }
 
@@ -570,62 +593,65 @@ __global__ __launch_bounds__(kThreads) void k_props(const double* __restrict__ T
 // (PlaneRing, stencil_grid.h) and marches through a run of planes of its 64 x 4
 // tile, as k_momentum (at 384x256x192: 0.240 -> 0.230 ms; the per-thread
 // version served its 14 neighbour reads per point from L1 and L2), and
-// loads divjac one plane ahead (-> 0.212 ms).  Same expressions on the same
-// values.
+// loads divjac one plane ahead (-> 0.212 ms; with no conditional load and one
+// barrier a plane -> 0.187).  Same expressions on the same values.
 __global__ __launch_bounds__(kThreads) void k_rhs_energy(const double* __restrict__ T,
                                                          const double* __restrict__ cond,
                                                          const double* __restrict__ divjac,
                                                          double* __restrict__ RHS, double* __restrict__ dvn,
                                                          const int* __restrict__ bot, const int* __restrict__ top,
                                                          Grid g, BandGrid bg, Geom G, Phys p) {
-    __shared__ double sF[2][3][kRingP];
+    __shared__ double sF[2][kRingSlots][kRingP];
     int i0, j0, k0, k1;
     if (!ring_tile(bg, g.ny, i0, j0, k0, k1)) return;
-    const int i = i0 + (int)threadIdx.x, j = j0 + (int)threadIdx.y;
-    const bool active = i < g.nx && j < g.nz;
     const double* fields[2] = {T, cond};
     PlaneRing<2> ring(sF, fields, i0, j0, g.nx, g.nz);
     ring.prime(k0);
-    const int e0 = ring_point();
+    const int row = tile_row(), j = j0 + row;
+    if (j >= g.nz) {
+        ring.stage(k0, k1);
+        return;
+    }
+    const int i = min(i0 + (int)threadIdx.x, g.nx - 1);
+    const int e0 = (row + 1) * kRingX + (i - i0) + 1;
     // the column's rough-wall slab (plane-independent) and divjac one plane
     // ahead, so that no step waits for a load of its own
     int cb = -1, ct = g.ny;
-    if (bot != nullptr && active) {
+    if (bot != nullptr) {
         const long col = (long)i + (long)g.nx * j;
         cb = bot[col];
         ct = top[col];
     }
-    double djn = active ? divjac[g.at(i, j, k0)] : 0.0;
+    double djn = divjac[g.at(i, j, k0)];
     for (int kk = k0; kk < k1; ++kk) {
-        ring.put(kk + 1);  // the slot of plane kk - 2, free since the last barrier
-        __syncthreads();
-        if (kk + 2 <= k1) ring.fetch(kk + 2);  // in flight during this step's arithmetic
+        ring.put(kk + 1);
         const double djac = djn;
-        if (active && kk + 1 < k1) djn = divjac[g.at(i, j, kk + 1)];
-        if (active) {
-            const int sm = (kk + 2) % 3, s0 = kk % 3, sp = (kk + 1) % 3;
-            auto slot = [&](int dk) { return dk < 0 ? sm : (dk > 0 ? sp : s0); };
-            auto t = [&](int di, int dj, int dk) { return sF[0][slot(dk)][e0 + di + dj * kRingX]; };
-            auto q = [&](int di, int dj, int dk) { return sF[1][slot(dk)][e0 + di + dj * kRingX]; };
-            const long c = g.at(i, j, kk);
-            const long o = (long)i + (long)g.nx * ((long)j + (long)g.nz * kk);
-            const double Ra = G.ruw[3 * kk], Rb = G.ruw[3 * kk + 1], Rc = G.ruw[3 * kk + 2];
-            const double R2a = G.ruw2[3 * kk], R2b = G.ruw2[3 * kk + 1], R2c = G.ruw2[3 * kk + 2];
-            const double d2tx = ((t(1, 0, 0) - 2 * t(0, 0, 0)) + t(-1, 0, 0)) * p.idx2;
-            const double d2tz = ((t(0, 1, 0) - 2 * t(0, 0, 0)) + t(0, -1, 0)) * p.idz2;
-            const double d2ty = (t(0, 0, -1) * R2a + t(0, 0, 0) * R2b) + t(0, 0, 1) * R2c;
-            const double grad =
-                (((q(1, 0, 0) - q(-1, 0, 0)) * p.idx__2) * ((t(1, 0, 0) - t(-1, 0, 0)) * p.idx__2) +
-                 ((q(0, 1, 0) - q(0, -1, 0)) * p.idz__2) * ((t(0, 1, 0) - t(0, -1, 0)) * p.idz__2)) +
-                ((q(0, 0, -1) * Ra + q(0, 0, 0) * Rb) + q(0, 0, 1) * Rc) *
-                    ((t(0, 0, -1) * Ra + t(0, 0, 0) * Rb) + t(0, 0, 1) * Rc);
-            const double rhs = (q(0, 0, 0) * ((d2tx + d2tz) + d2ty) + grad) + p.Sq;
-            RHS[o] = rhs;
-            double dn = djac * rhs;
-            if (kk <= cb || kk >= ct) dn = 0.0;
-            dvn[c] = dn;
-        }
-        __syncthreads();  // slot (kk + 2) % 3 is restaged next
+        __syncthreads();
+        ring.fetch(min(kk + 2, k1));  // in flight during this step's arithmetic
+        djn = divjac[g.at(i, j, min(kk + 1, k1 - 1))];
+        const int sm = ring_slot(kk - 1), s0 = ring_slot(kk), sp = ring_slot(kk + 1);
+        auto slot = [&](int dk) { return dk < 0 ? sm : (dk > 0 ? sp : s0); };
+        auto t = [&](int di, int dj, int dk) { return sF[0][slot(dk)][e0 + di + dj * kRingX]; };
+        auto q = [&](int di, int dj, int dk) { return sF[1][slot(dk)][e0 + di + dj * kRingX]; };
+        const long c = g.at(i, j, kk);
+        const long o = (long)i + (long)g.nx * ((long)j + (long)g.nz * kk);
+        const double Ra = uniform_load(G.ruw, 3 * kk), Rb = uniform_load(G.ruw, 3 * kk + 1),
+                     Rc = uniform_load(G.ruw, 3 * kk + 2);
+        const double R2a = uniform_load(G.ruw2, 3 * kk), R2b = uniform_load(G.ruw2, 3 * kk + 1),
+                     R2c = uniform_load(G.ruw2, 3 * kk + 2);
+        const double d2tx = ((t(1, 0, 0) - 2 * t(0, 0, 0)) + t(-1, 0, 0)) * p.idx2;
+        const double d2tz = ((t(0, 1, 0) - 2 * t(0, 0, 0)) + t(0, -1, 0)) * p.idz2;
+        const double d2ty = (t(0, 0, -1) * R2a + t(0, 0, 0) * R2b) + t(0, 0, 1) * R2c;
+        const double grad =
+            (((q(1, 0, 0) - q(-1, 0, 0)) * p.idx__2) * ((t(1, 0, 0) - t(-1, 0, 0)) * p.idx__2) +
+             ((q(0, 1, 0) - q(0, -1, 0)) * p.idz__2) * ((t(0, 1, 0) - t(0, -1, 0)) * p.idz__2)) +
+            ((q(0, 0, -1) * Ra + q(0, 0, 0) * Rb) + q(0, 0, 1) * Rc) *
+                ((t(0, 0, -1) * Ra + t(0, 0, 0) * Rb) + t(0, 0, 1) * Rc);
+        const double rhs = (q(0, 0, 0) * ((d2tx + d2tz) + d2ty) + grad) + p.Sq;
+        RHS[o] = rhs;
+        double dn = djac * rhs;
+        if (kk <= cb || kk >= ct) dn = 0.0;
+        dvn[c] = dn;
     }
 }
 

@@ -101,7 +101,7 @@ __device__ __forceinline__ double rfac(double rho_min, double nb, double rc) {
 // points each, so they are staged in LDS: a workgroup owns a 64 x 4 (i, j)
 // tile and marches through a run of planes, keeping planes k-1, k,
 // k+1 of the three fields (tile plus one halo point in x and z) in a ring of
-// three LDS slots and loading one new plane per step (issued before the
+// LDS slots and loading one new plane per step (issued before the
 // step's arithmetic), so each of their values is read about once instead
 // of by every neighbouring thread (0.36 -> 0.28 ms at 384x256x192; the
 // per-thread version made 6.3 L1 requests per point).
@@ -112,46 +112,62 @@ __global__ __launch_bounds__(kTileX * kTileZ) void k_rhs_varprop(
     const double* __restrict__ rho_min_p, Halo h, BandGrid bg, double inv_dtmax, double inv_dx, double inv_dz,
     double inv_dx2, double inv_dz2) {
 #pragma clang fp contract(off)
-    __shared__ double sF[3][3][kRingP];  // P_now, P_old, rho
+    __shared__ double sF[3][kRingSlots][kRingP];  // P_now, P_old, rho
     int i0, j0, k0, k1;
     if (!ring_tile(bg, h.ny, i0, j0, k0, k1)) return;
-    const int i = i0 + (int)threadIdx.x, j = j0 + (int)threadIdx.y;
-    const bool active = i < h.nx && j < h.nz;
-    const long sz = h.sz(), sy = h.sy();
     const double* fields[3] = {Pn, Po, rho};
     PlaneRing<3> ring(sF, fields, i0, j0, h.nx, h.nz);
     ring.prime(k0);
+    // lanes past the last column repeat its point (same loads, same stores)
+    const int row = tile_row(), j = j0 + row;
+    if (j >= h.nz) {
+        ring.stage(k0, k1);
+        return;
+    }
+    const int i = min(i0 + (int)threadIdx.x, h.nx - 1);
+    const int e0 = (row + 1) * kRingX + (i - i0) + 1;
+    const long sz = h.sz(), sy = h.sy();
+    // the point's velocities and div_now, loaded a plane ahead; V_hat(k + 1) is
+    // the next step's V_hat(k)
+    struct Ahead {
+        double u, ux, w, wz, vy, d;
+    };
+    auto ahead = [&](int k) {
+        const long c = h.at(i, j, k);
+        return Ahead{Uh[c], Uh[c + 1], Wh[c], Wh[c + sz], Vh[c + sy], div_now[c]};
+    };
+    double v = Vh[h.at(i, j, k0)];
+    Ahead nxt = ahead(k0);
     const double rho_min = *rho_min_p;
-    const int e0 = ring_point();
     for (int k = k0; k < k1; ++k) {
-        ring.put(k + 1);  // the slot of plane k - 2, free since the last barrier
+        ring.put(k + 1);
+        const Ahead a = nxt;
         __syncthreads();
-        if (k + 2 <= k1) ring.fetch(k + 2);  // in flight during this step's arithmetic
-        if (active) {
-            const int sm = (k + 2) % 3, s0 = k % 3, sp = (k + 1) % 3;
-            const long c = h.at(i, j, k);
-            auto ps = [&](int slot, int e) { return 2 * sF[0][slot][e] - sF[1][slot][e]; };
-            auto rh = [&](int slot, int e) { return sF[2][slot][e]; };
-            const double Ps_00 = ps(s0, e0);
-            const double Ps_xp = ps(s0, e0 + 1), Ps_xm = ps(s0, e0 - 1);
-            const double Ps_zp = ps(s0, e0 + kRingX), Ps_zm = ps(s0, e0 - kRingX);
-            const double Ps_yp = ps(sp, e0), Ps_ym = ps(sm, e0);
-            const double rc = rh(s0, e0);
-            const double rho_xp = rfac(rho_min, rh(s0, e0 + 1), rc), rho_xm = rfac(rho_min, rh(s0, e0 - 1), rc);
-            const double rho_zp = rfac(rho_min, rh(s0, e0 + kRingX), rc);
-            const double rho_zm = rfac(rho_min, rh(s0, e0 - kRingX), rc);
-            const double rho_yp = rfac(rho_min, rh(sp, e0), rc), rho_ym = rfac(rho_min, rh(sm, e0), rc);
-            const double idy = inv_dy_p[k];
-            const double t1 = inv_dtmax * (((Uh[c + 1] - Uh[c]) * inv_dx + (Wh[c + sz] - Wh[c]) * inv_dz) +
-                                           (Vh[c + sy] - Vh[c]) * idy) * rho_min;
-            const double t2 = inv_dtmax * rho_min * div_now[c];
-            const double t3 = ((rho_xp * (Ps_xp - Ps_00) - rho_xm * (Ps_00 - Ps_xm)) * inv_dx2 +
-                               (rho_zp * (Ps_zp - Ps_00) - rho_zm * (Ps_00 - Ps_zm)) * inv_dz2) +
-                              (rho_yp * (Ps_yp - Ps_00) * inv_dy_p_pad[k + 1] -
-                               rho_ym * (Ps_00 - Ps_ym) * inv_dy_p_pad[k]) * idy;
-            P[(long)i + (long)h.nx * ((long)j + (long)h.nz * k)] = (t1 - t2) + t3;
-        }
-        __syncthreads();  // slot (k + 2) % 3 is restaged next
+        // in flight during this step's arithmetic
+        ring.fetch(min(k + 2, k1));
+        nxt = ahead(min(k + 1, k1 - 1));
+        const int sm = ring_slot(k - 1), s0 = ring_slot(k), sp = ring_slot(k + 1);
+        auto ps = [&](int slot, int e) { return 2 * sF[0][slot][e] - sF[1][slot][e]; };
+        auto rh = [&](int slot, int e) { return sF[2][slot][e]; };
+        const double Ps_00 = ps(s0, e0);
+        const double Ps_xp = ps(s0, e0 + 1), Ps_xm = ps(s0, e0 - 1);
+        const double Ps_zp = ps(s0, e0 + kRingX), Ps_zm = ps(s0, e0 - kRingX);
+        const double Ps_yp = ps(sp, e0), Ps_ym = ps(sm, e0);
+        const double rc = rh(s0, e0);
+        const double rho_xp = rfac(rho_min, rh(s0, e0 + 1), rc), rho_xm = rfac(rho_min, rh(s0, e0 - 1), rc);
+        const double rho_zp = rfac(rho_min, rh(s0, e0 + kRingX), rc);
+        const double rho_zm = rfac(rho_min, rh(s0, e0 - kRingX), rc);
+        const double rho_yp = rfac(rho_min, rh(sp, e0), rc), rho_ym = rfac(rho_min, rh(sm, e0), rc);
+        const double idy = uniform_load(inv_dy_p, k);
+        const double t1 =
+            inv_dtmax * (((a.ux - a.u) * inv_dx + (a.wz - a.w) * inv_dz) + (a.vy - v) * idy) * rho_min;
+        const double t2 = inv_dtmax * rho_min * a.d;
+        const double t3 = ((rho_xp * (Ps_xp - Ps_00) - rho_xm * (Ps_00 - Ps_xm)) * inv_dx2 +
+                           (rho_zp * (Ps_zp - Ps_00) - rho_zm * (Ps_00 - Ps_zm)) * inv_dz2) +
+                          (rho_yp * (Ps_yp - Ps_00) * uniform_load(inv_dy_p_pad, k + 1) -
+                           rho_ym * (Ps_00 - Ps_ym) * uniform_load(inv_dy_p_pad, k)) * idy;
+        P[(long)i + (long)h.nx * ((long)j + (long)h.nz * k)] = (t1 - t2) + t3;
+        v = a.vy;
     }
 }
 

@@ -13,6 +13,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cstdint>
+
 #include "fft_ct.h"
 
 namespace dnsp {
@@ -64,15 +66,24 @@ __device__ __forceinline__ bool band_point(const BandGrid& b, int& i, int& j, in
     return i < b.nx && j < b.nz;
 }
 
-// Ring of three planes of NF halo fields in LDS, for a workgroup of
+// Ring of four planes of NF halo fields in LDS, for a workgroup of
 // kTileX x kTileZ threads that owns one (i, j) tile and marches through a run
 // of planes in k.  A slot holds one plane of the tile plus one halo point on
 // each side in x and z (kRingX x kRingZ values, point (i, j) of the tile at
-// (j + 1) * kRingX + i + 1); plane kp (-1..ny) lives in slot (kp + 3) % 3.
+// (j + 1) * kRingX + i + 1); plane kp (-1..ny) lives in slot kp & 3.
 // Each thread stages halo-tile points tid and tid + 256: fetch(kp) loads
 // plane kp into registers, put(kp) stores them to the slot, so the loads of
 // the next plane can be issued before a step's arithmetic.  Fields are the
 // reference's halo arrays ((nx+2)(nz+2)(ny+2), x fastest).
+//
+// Four slots, so that a step needs one barrier: plane k + 2 goes to the slot
+// of plane k - 2, which nobody reads once the barrier of step k - 1 is passed.
+//
+// No load here is conditional.  Vector memory returns in order and the compiler
+// counts what was issued since, over all paths: behind a branch that might skip
+// a load it waits for everything outstanding, the step's prefetches and the last
+// step's stores included.  Threads past the halo tile and points past the grid's
+// halo repeat a valid address instead (and the value stored with it).
 constexpr int kRingX = kTileX + 2, kRingZ = kTileZ + 2, kRingP = kRingX * kRingZ;
 
 // Band order over tiles and runs of planes (an XCD walks the tiles of its band
@@ -107,43 +118,43 @@ __device__ __forceinline__ bool ring_tile(const BandGrid& b, int ny, int& i0, in
     return j0 < b.nz;
 }
 
+constexpr int kRingSlots = 4;
+__device__ __forceinline__ int ring_slot(int kp) { return kp & (kRingSlots - 1); }
+
 template <int NF>
 struct PlaneRing {
     static constexpr int kNT = kTileX * kTileZ;
     static_assert(kRingP <= 2 * kNT, "two staged points per thread");
-    double (*lds)[3][kRingP];
+    double (*lds)[kRingSlots][kRingP];
     const double* f[NF];
     long go[2], sy;
-    bool ok[2];
+    int le[2];
     double r[NF][2];
-    int tid;
 
-    // Tile at (i0, j0) of an nx x nz x ny grid; lds points to NF x 3 slots.
-    __device__ __forceinline__ PlaneRing(double (*lds_)[3][kRingP], const double* const* fields, int i0, int j0,
-                                         int nx, int nz)
+    // Tile at (i0, j0) of an nx x nz x ny grid; lds points to NF x 4 slots.
+    __device__ __forceinline__ PlaneRing(double (*lds_)[kRingSlots][kRingP], const double* const* fields, int i0,
+                                         int j0, int nx, int nz)
         : lds(lds_) {
         for (int q = 0; q < NF; ++q) f[q] = fields[q];
-        tid = (int)threadIdx.y * kTileX + (int)threadIdx.x;
+        const int tid = (int)threadIdx.y * kTileX + (int)threadIdx.x;
         const long sz = nx + 2;
         sy = sz * (nz + 2);
         for (int u = 0; u < 2; ++u) {
-            const int e = tid + u * kNT;
+            const int e = min(tid + u * kNT, kRingP - 1);
             const int rr = e / kRingX, qq = e - rr * kRingX;
-            const int gi = i0 - 1 + qq, gj = j0 - 1 + rr;
-            ok[u] = e < kRingP && gi <= nx && gj <= nz;
-            go[u] = ok[u] ? (long)(gi + 1) + sz * (long)(gj + 1) + sy : 0;  // plane 0
+            const int gi = min(i0 - 1 + qq, nx), gj = min(j0 - 1 + rr, nz);
+            le[u] = e;
+            go[u] = (long)(gi + 1) + sz * (long)(gj + 1) + sy;  // plane 0
         }
     }
     __device__ __forceinline__ void fetch(int kp) {
         for (int u = 0; u < 2; ++u)
-            if (ok[u])
-                for (int q = 0; q < NF; ++q) r[q][u] = f[q][go[u] + (long)kp * sy];
+            for (int q = 0; q < NF; ++q) r[q][u] = f[q][go[u] + (long)kp * sy];
     }
     __device__ __forceinline__ void put(int kp) {
-        const int slot = (kp + 3) % 3;
+        const int slot = ring_slot(kp);
         for (int u = 0; u < 2; ++u)
-            if (ok[u])
-                for (int q = 0; q < NF; ++q) lds[q][slot][tid + u * kNT] = r[q][u];
+            for (int q = 0; q < NF; ++q) lds[q][slot][le[u]] = r[q][u];
     }
     // Planes k0 - 1 and k0 into their slots and k0 + 1 into the registers, the
     // loads of all three in flight together.
@@ -151,18 +162,32 @@ struct PlaneRing {
         double a[2][NF][2];
         for (int h = 0; h < 2; ++h)
             for (int u = 0; u < 2; ++u)
-                for (int q = 0; q < NF; ++q) a[h][q][u] = ok[u] ? f[q][go[u] + (long)(k0 - 1 + h) * sy] : 0.0;
+                for (int q = 0; q < NF; ++q) a[h][q][u] = f[q][go[u] + (long)(k0 - 1 + h) * sy];
         fetch(k0 + 1);
         for (int h = 0; h < 2; ++h) {
-            const int slot = (k0 + 2 + h) % 3;
+            const int slot = ring_slot(k0 - 1 + h);
             for (int u = 0; u < 2; ++u)
-                if (ok[u])
-                    for (int q = 0; q < NF; ++q) lds[q][slot][tid + u * kNT] = a[h][q][u];
+                for (int q = 0; q < NF; ++q) lds[q][slot][le[u]] = a[h][q][u];
+        }
+    }
+    // The march of a wave that owns no row of the grid: it only stages.
+    __device__ __forceinline__ void stage(int k0, int k1) {
+        for (int k = k0; k < k1; ++k) {
+            put(k + 1);
+            __syncthreads();
+            fetch(min(k + 2, k1));
         }
     }
 };
 
-// This thread's point in a ring slot.
-__device__ __forceinline__ int ring_point() { return ((int)threadIdx.y + 1) * kRingX + (int)threadIdx.x + 1; }
+// This wave's row of the tile (a wave is one row), as a uniform value.
+__device__ __forceinline__ int tile_row() { return __builtin_amdgcn_readfirstlane((int)threadIdx.y); }
+
+// p[i] for a uniform i of data no kernel in flight writes, as a scalar load: a
+// vector load would be waited for in order behind the step's prefetches.
+__device__ __forceinline__ double uniform_load(const double* p, int i) {
+    typedef const double __attribute__((address_space(4))) * ConstPtr;
+    return ((ConstPtr)(uintptr_t)p)[i];
+}
 
 }  // namespace dnsp
