@@ -115,10 +115,11 @@ __global__ void k_div_finish(double* D, Grid g) {
 // (mod_cfd_subroutines.f90:147-354).  u, v, w, m(di, dj, dk) return U, V,
 // W, mu at (i + di, j + dj, k + dk); r, dv, b likewise rho, div_now and the
 // buoyancy field (read at the point and at (-1, 0, 0), (0, -1, 0), (0, 0, -1)).
-template <bool VARPROP, class AU, class AV, class AW, class AM, class AR, class AD, class AB>
+template <bool VARPROP, bool NT, class AU, class AV, class AW, class AM, class AR, class AD, class AB>
 __device__ __forceinline__ void momentum_point(
-    const AU& u, const AV& v, const AW& w, const AM& m, const AR& r, const AD& dv, const AB& b, long c, long o, int k, double ru_old,
-    double rv_old, double rw_old, double* __restrict__ Ru_old, double* __restrict__ Rv_old, double* __restrict__ Rw_old,
+    const AU& u, const AV& v, const AW& w, const AM& m, const AR& r, const AD& dv, const AB& b, long c, long o, int k,
+    double ru_old, double rv_old, double rw_old, double* __restrict__ Ru_old, double* __restrict__ Rv_old,
+    double* __restrict__ Rw_old,
     double* __restrict__ U_hat, double* __restrict__ V_hat, double* __restrict__ W_hat, const Grid& g,
     const Geom& G, const Phys& p, int kmin_Vhat) {
     const double idx = p.idx, idz = p.idz, idx2 = p.idx2, idz2 = p.idz2, idx__2 = p.idx__2, idz__2 = p.idz__2;
@@ -181,10 +182,10 @@ __device__ __forceinline__ void momentum_point(
                      (0.5 * (r(0, -1, 0) + r(0, 0, 0)));
             }
         }
-        U_hat[c] = u(0, 0, 0) + p.dt * (1.5 * Ru - 0.5 * ru_old);
-        W_hat[c] = w(0, 0, 0) + p.dt * (1.5 * Rw - 0.5 * rw_old);
-        Ru_old[o] = Ru;
-        Rw_old[o] = Rw;
+        stream_store<NT>(U_hat + c, u(0, 0, 0) + p.dt * (1.5 * Ru - 0.5 * ru_old));
+        stream_store<NT>(W_hat + c, w(0, 0, 0) + p.dt * (1.5 * Rw - 0.5 * rw_old));
+        stream_store<NT>(Ru_old + o, Ru);
+        stream_store<NT>(Rw_old + o, Rw);
     }
     if (k < kmin_Vhat) return;
     {
@@ -217,8 +218,8 @@ __device__ __forceinline__ void momentum_point(
             const double visc = (((0.5 * (m(0, 0, -1) + m(0, 0, 0))) * D + E * Fx) + Gt * H) + I * J;
             Rv = ((-conv + visc) + p.Gb_y * (0.5 * (b(0, 0, 0) + b(0, 0, -1)))) / (0.5 * (r(0, 0, -1) + r(0, 0, 0)));
         }
-        V_hat[c] = v(0, 0, 0) + p.dt * (1.5 * Rv - 0.5 * rv_old);
-        Rv_old[o] = Rv;
+        stream_store<NT>(V_hat + c, v(0, 0, 0) + p.dt * (1.5 * Rv - 0.5 * rv_old));
+        stream_store<NT>(Rv_old + o, Rv);
     }
 }
 
@@ -234,9 +235,9 @@ __device__ __forceinline__ void momentum_point(
 // order and a wait for a late one waits for the whole prefetch (the version with
 // loads inside the step waited for everything outstanding five times a plane:
 // 683 us at 384x192x256, 3.9 TB/s over 93 + 48 B/pt from beyond L2; now 565 us,
-// 4.7 TB/s).  203 VGPRs, two waves per SIMD; capped for three: 577 us; two planes
+// 4.7 TB/s; stored past the caches 555).  200 VGPRs, two waves per SIMD; capped for three: 577 us; two planes
 // of the ring in flight instead of one: 562, and 2% more on small grids.
-template <bool VARPROP>
+template <bool VARPROP, bool NT>
 __global__ __launch_bounds__(kThreads) void k_momentum(
     const double* __restrict__ U, const double* __restrict__ V, const double* __restrict__ W,
     const double* __restrict__ mu, const double* __restrict__ rho, const double* __restrict__ dvn,
@@ -310,7 +311,7 @@ __global__ __launch_bounds__(kThreads) void k_momentum(
         auto lr = [&](int di, int dj, int dk) { return at(0, di, dj, dk); };
         auto ld = [&](int di, int dj, int dk) { return at(1, di, dj, dk); };
         auto lb = [&](int di, int dj, int dk) { return at(2, di, dj, dk); };
-        momentum_point<VARPROP>(lu, lv, lw, lm, lr, ld, lb, g.at(i, j, k),
+        momentum_point<VARPROP, NT>(lu, lv, lw, lm, lr, ld, lb, g.at(i, j, k),
                                 (long)i + (long)g.nx * ((long)j + (long)g.nz * k), k, a.old[0], a.old[1], a.old[2],
                                 Ru_old, Rv_old, Rw_old, U_hat, V_hat, W_hat, g, G, p, kmin_Vhat);
 #pragma unroll
@@ -469,8 +470,11 @@ __device__ __forceinline__ double seg_eval(const double* seg, int sgi, double T)
 // searches read LDS.
 constexpr int kMaxSegments = 1024;  // 48 KB of LDS, plus 6 KB of bucket tables (merged tables: up to 64 KB in all)
 
-// IDX32: the padded field has fewer than 2^31 points (32-bit index split).
-template <bool ALL_CUBIC, bool IDX32>
+// IDX32: the padded field has fewer than 2^31 points (32-bit index split); NT:
+// stream_store.  Bound by its eight store streams (at 384x192x256 77 B/pt from and to
+// beyond L2: 352 us through the caches, 310 past them, 4.7 TB/s; loads without a
+// condition a pair ahead instead of two pairs ahead took 128 VGPRs and 373 us).
+template <bool ALL_CUBIC, bool IDX32, bool NT>
 __global__ __launch_bounds__(kThreads) void k_props(const double* __restrict__ T, double* __restrict__ T_ext,
                                                     double* __restrict__ enth, double* __restrict__ rho,
                                                     double* __restrict__ mu, double* __restrict__ cond,
@@ -574,9 +578,10 @@ __global__ __launch_bounds__(kThreads) void k_props(const double* __restrict__ T
         double o0[7], o1[7];
         eval(te0, o0);
         eval(te1, o1);
-        reinterpret_cast<double2*>(out[0])[p] = make_double2(te0, te1);
+        stream_store<NT>(reinterpret_cast<double2*>(out[0]) + p, make_double2(te0, te1));
 #pragma unroll
-        for (int q = 0; q < 7; ++q) reinterpret_cast<double2*>(out[q + 1])[p] = make_double2(o0[q], o1[q]);
+        for (int q = 0; q < 7; ++q)
+            stream_store<NT>(reinterpret_cast<double2*>(out[q + 1]) + p, make_double2(o0[q], o1[q]));
     }
     if ((n & 1) && blockIdx.x == 0 && threadIdx.x == 0) {
         const double te = wall_te(n - 1, T[n - 1]);
@@ -594,7 +599,8 @@ __global__ __launch_bounds__(kThreads) void k_props(const double* __restrict__ T
 // tile, as k_momentum (at 384x256x192: 0.240 -> 0.230 ms; the per-thread
 // version served its 14 neighbour reads per point from L1 and L2), and
 // loads divjac one plane ahead (-> 0.212 ms; with no conditional load and one
-// barrier a plane -> 0.187).  Same expressions on the same values.
+// barrier a plane -> 0.187; stored past the caches 0.183).  Same expressions on the same values.
+template <bool NT>
 __global__ __launch_bounds__(kThreads) void k_rhs_energy(const double* __restrict__ T,
                                                          const double* __restrict__ cond,
                                                          const double* __restrict__ divjac,
@@ -648,10 +654,10 @@ __global__ __launch_bounds__(kThreads) void k_rhs_energy(const double* __restric
             ((q(0, 0, -1) * Ra + q(0, 0, 0) * Rb) + q(0, 0, 1) * Rc) *
                 ((t(0, 0, -1) * Ra + t(0, 0, 0) * Rb) + t(0, 0, 1) * Rc);
         const double rhs = (q(0, 0, 0) * ((d2tx + d2tz) + d2ty) + grad) + p.Sq;
-        RHS[o] = rhs;
+        stream_store<NT>(RHS + o, rhs);
         double dn = djac * rhs;
         if (kk <= cb || kk >= ct) dn = 0.0;
-        dvn[c] = dn;
+        stream_store<NT>(dvn + c, dn);
     }
 }
 
@@ -1130,15 +1136,12 @@ int dnsp_predictor_enqueue(dnsp_predictor* pr, void* stream) {
     // 3. momentum predictor
     double* mu = pr->f[DNSP_PRED_MU];
     double* buoy = pr->f[DNSP_PRED_BUOY];
-    if (vp)
-        k_momentum<true><<<gridr, blk3, 0, st>>>(U, V, W, mu, rho, dvn, buoy, pr->f[DNSP_PRED_RU_OLD],
-                                                     pr->f[DNSP_PRED_RV_OLD], pr->f[DNSP_PRED_RW_OLD], Uh, Vh, Wh, g,
-                                                     br, pr->G, pr->p, pr->kmin_Vhat);
-    else
-        k_momentum<false><<<gridr, blk3, 0, st>>>(U, V, W, nullptr, nullptr, nullptr, nullptr,
-                                                      pr->f[DNSP_PRED_RU_OLD], pr->f[DNSP_PRED_RV_OLD],
-                                                      pr->f[DNSP_PRED_RW_OLD], Uh, Vh, Wh, g, br, pr->G, pr->p,
-                                                      pr->kmin_Vhat);
+    const bool past = streams_past(g.total(), 6);
+    auto km = vp ? (past ? k_momentum<true, true> : k_momentum<true, false>)
+                 : (past ? k_momentum<false, true> : k_momentum<false, false>);
+    km<<<gridr, blk3, 0, st>>>(U, V, W, vp ? mu : nullptr, vp ? rho : nullptr, vp ? dvn : nullptr, vp ? buoy : nullptr,
+                               pr->f[DNSP_PRED_RU_OLD], pr->f[DNSP_PRED_RV_OLD], pr->f[DNSP_PRED_RW_OLD], Uh, Vh, Wh, g,
+                               br, pr->G, pr->p, pr->kmin_Vhat);
     // 4. temperature
     if (vp)
         k_temp_rhs<true><<<grid3, blk3, 0, st>>>(T, U, V, W, rho, pr->f[DNSP_PRED_CP],
@@ -1166,8 +1169,11 @@ int dnsp_predictor_enqueue(dnsp_predictor* pr, void* stream) {
         const int nbp = std::min(blocks_for(g.total()), 2048);
         const bool all_cubic = pr->ml.m >= 0;
         const bool idx32 = g.total() < (1L << 31);
-        auto kp = all_cubic ? (idx32 ? k_props<true, true> : k_props<true, false>)
-                            : (idx32 ? k_props<false, true> : k_props<false, false>);
+        const bool past = streams_past(g.total(), 8);
+        auto kp = all_cubic ? (!idx32 ? k_props<true, false, true>
+                                      : (past ? k_props<true, true, true> : k_props<true, true, false>))
+                            : (!idx32 ? k_props<false, false, true>
+                                      : (past ? k_props<false, true, true> : k_props<false, true, false>));
         const size_t lds = sizeof(double) * 6 * nseg +
                            (all_cubic ? sizeof(double) * pr->ml.m + sizeof(int) * (6 * (pr->ml.m + 1) + kMergedBuckets)
                                       : sizeof(int) * Q_N * kBuckets);
@@ -1182,7 +1188,8 @@ int dnsp_predictor_enqueue(dnsp_predictor* pr, void* stream) {
             if (!rc) rc = dnsp_set_val_slice(T, g.nx, g.nz, g.ny, -1, -1, wl[7], vs);
             if (rc) return rc;
         }
-        k_rhs_energy<<<gridr, blk3, 0, st>>>(T, pr->f[DNSP_PRED_COND], pr->f[DNSP_PRED_DIVJAC],
+        auto ke = streams_past(g.total(), 2) ? k_rhs_energy<true> : k_rhs_energy<false>;
+        ke<<<gridr, blk3, 0, st>>>(T, pr->f[DNSP_PRED_COND], pr->f[DNSP_PRED_DIVJAC],
                                                  pr->f[DNSP_PRED_RHS_ENERGY], dvn, pr->d_bot[3], pr->d_top[3], g, br,
                                                  pr->G, pr->p);
         k_div_finish<<<blocks_for(2 * g.sy() + per_plane * g.ny), kThreads, 0, st>>>(dvn, g);

@@ -180,6 +180,31 @@ struct PlaneRing {
     }
 };
 
+// Store past the caches (NT) or through them.  A kernel that writes several
+// fields whose next reader is a whole pass away only evicts with them what
+// others will read: at 384x192x256 (155 MB a field), through / past: eight
+// streams of a copy 302 / 225 us, the property kernel 352 / 310, momentum 568 /
+// 555, and the next kernels gain what stays cached (the minimum of rho 42 / 30).
+// Where a kernel's outputs fit the cache they are read back from it: at 96x48x65
+// the whole time step takes 120.5 / 124.5.
+template <bool NT>
+__device__ __forceinline__ void stream_store(double* p, double v) {
+    if constexpr (NT) __builtin_nontemporal_store(v, p);
+    else *p = v;
+}
+template <bool NT>
+__device__ __forceinline__ void stream_store(double2* p, double2 v) {
+    if constexpr (NT) {
+        typedef double Pair __attribute__((ext_vector_type(2)));
+        __builtin_nontemporal_store(Pair{v.x, v.y}, reinterpret_cast<Pair*>(p));
+    } else {
+        *p = v;
+    }
+}
+// Whether a kernel that writes nout fields of `points` values stores past the
+// caches: more than the 256 MB of the last one.
+inline bool streams_past(long points, int nout) { return points * nout * (long)sizeof(double) > (256L << 20); }
+
 // This wave's row of the tile (a wave is one row), as a uniform value.
 __device__ __forceinline__ int tile_row() { return __builtin_amdgcn_readfirstlane((int)threadIdx.y); }
 

@@ -43,3 +43,11 @@ def test_rhs_varprop_tile_edges_bitexact(cuda, nx, nz, ny):
                                  3.5 ** 2, 2.25 ** 2, rm)
     torch.cuda.synchronize()
     assert np.array_equal(P.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("nx,nz,ny", [(512, 128, 100), (512, 128, 257)])
+def test_predictor_stores_past_the_caches(cuda, nx, nz, ny):
+    """Sizes from which the momentum and property kernels (6.8 M padded points)
+    and also the energy right-hand side (17 M) store past the caches."""
+    TP.say("ring tiles large", nx, nz, ny)
+    TP.test_predictor_matches_oracle(cuda, "nicoud", nx, nz, ny)
