@@ -11,6 +11,27 @@
 
 namespace dnsp {
 
+// Load past the caches (NT) or through them, for the blocked solve's transforms: a
+// stage reads every value once and overwrites the array it read two stages
+// later, so a line kept after its read only pushes out the stage's own output, which
+// the next stage reads.  us per solve, through / past: 384x192x256 290 / 268,
+// 512x256x256 539 / 481, 256x384x256 398 / 354, 768x384x384 1743 / 1728; no
+// difference where two fields fit the 256 MB cache (64x32x64, 256x128x192).  The
+// tridiagonal's loads make none.
+template <bool NT>
+__device__ __forceinline__ double2 stream_load(const double2* p) {
+    if constexpr (NT) {
+        typedef double Pair __attribute__((ext_vector_type(2)));
+        const Pair v = __builtin_nontemporal_load(reinterpret_cast<const Pair*>(p));
+        return make_double2(v.x, v.y);
+    } else {
+        return *p;
+    }
+}
+// The z transforms of 512 points keep ordinary loads: 384x512x256 takes 846 us with
+// them, 874 past the caches (z forward alone at 512x512x288 267 and 305).
+constexpr bool z_loads_past(int n) { return n != 512; }
+
 // FFT kernel variants: (complex elements per workgroup tile, threads), one
 // table per direction.  The tuner picks one per direction and handle.  x
 // variant 0 is one complex line (two real lines) per workgroup at nx = 768:
@@ -78,7 +99,7 @@ __device__ __forceinline__ void xfwd_body(const double* P, double* S, long nline
     for (int q = 0; q < NL; ++q) {
         const int e = (int)threadIdx.x + q * NT;
         const int r = (2 * e) / N;
-        v[q] = ((G * N % NT == 0 || e < G * N) && l0 + r < nlines) ? src[e] : make_double2(0.0, 0.0);
+        v[q] = ((G * N % NT == 0 || e < G * N) && l0 + r < nlines) ? stream_load<XB>(src + e) : make_double2(0.0, 0.0);
     }
 #pragma unroll
     for (int q = 0; q < NL; ++q) {
@@ -163,7 +184,7 @@ __device__ __forceinline__ void xbwd_body(const double* S, double* P, long nline
             const int line = (2 * e) / N;
             const int off = 2 * e - line * N;
             const int ln = l0 + line < nlines ? line : 0;
-            v[q] = *reinterpret_cast<const double2*>(src + (long)ln * N + off);
+            v[q] = stream_load<true>(reinterpret_cast<const double2*>(src + (long)ln * N + off));
         }
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
@@ -533,7 +554,7 @@ __global__ __launch_bounds__(NT) void kt_zfwd_mm(const double* __restrict__ W, d
 #pragma unroll
     for (int q = 0; q < NL2; ++q) {
         const int e = (int)threadIdx.x + q * NT;
-        v[q] = (TOT2 % NT == 0 || e < TOT2) ? src[e] : make_double2(0.0, 0.0);
+        v[q] = (TOT2 % NT == 0 || e < TOT2) ? stream_load<z_loads_past(N)>(src + e) : make_double2(0.0, 0.0);
     }
 #pragma unroll
     for (int q = 0; q < NL2; ++q) {
@@ -587,8 +608,8 @@ __global__ __launch_bounds__(NT) void kt_zbwd_xl(const double* __restrict__ W, d
         const int tt = ee % TA;
         const int qq = ee / TA;
         const int qm = (qq == 0 || 2 * qq == N) ? qq : N - qq;
-        pu[q] = *reinterpret_cast<const double2*>(src + (size_t)qq * 16 + 2 * tt);
-        pi[q] = *reinterpret_cast<const double2*>(src + (size_t)qm * 16 + 2 * tt);
+        pu[q] = stream_load<z_loads_past(N)>(reinterpret_cast<const double2*>(src + (size_t)qq * 16 + 2 * tt));
+        pi[q] = stream_load<z_loads_past(N)>(reinterpret_cast<const double2*>(src + (size_t)qm * 16 + 2 * tt));
     }
 #pragma unroll
     for (int q = 0; q < NI; ++q) {
