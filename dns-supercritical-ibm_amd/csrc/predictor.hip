@@ -235,7 +235,7 @@ __device__ __forceinline__ void momentum_point(
 // order and a wait for a late one waits for the whole prefetch (the version with
 // loads inside the step waited for everything outstanding five times a plane:
 // 683 us at 384x192x256, 3.9 TB/s over 93 + 48 B/pt from beyond L2; now 565 us,
-// 4.7 TB/s; stored past the caches 555).  200 VGPRs, two waves per SIMD; capped for three: 577 us; two planes
+// 4.7 TB/s; the old R loaded and the outputs stored past the caches 550).  200 VGPRs, two waves per SIMD; capped for three: 577 us; two planes
 // of the ring in flight instead of one: 562, and 2% more on small grids.
 template <bool VARPROP, bool NT>
 __global__ __launch_bounds__(kThreads) void k_momentum(
@@ -278,9 +278,9 @@ __global__ __launch_bounds__(kThreads) void k_momentum(
                 a.z[q] = f[q][c - sz];
             }
         }
-        a.old[0] = Ru_old[o];
-        a.old[1] = Rv_old[o];
-        a.old[2] = Rw_old[o];
+        a.old[0] = stream_load<NT>(Ru_old + o);
+        a.old[1] = stream_load<NT>(Rv_old + o);
+        a.old[2] = stream_load<NT>(Rw_old + o);
         return a;
     };
     // rho, div_now and buoy at plane k - 1: carried from the step before
@@ -599,7 +599,7 @@ __global__ __launch_bounds__(kThreads) void k_props(const double* __restrict__ T
 // tile, as k_momentum (at 384x256x192: 0.240 -> 0.230 ms; the per-thread
 // version served its 14 neighbour reads per point from L1 and L2), and
 // loads divjac one plane ahead (-> 0.212 ms; with no conditional load and one
-// barrier a plane -> 0.187; stored past the caches 0.183).  Same expressions on the same values.
+// barrier a plane -> 0.187; past the caches 0.167).  Same expressions on the same values.
 template <bool NT>
 __global__ __launch_bounds__(kThreads) void k_rhs_energy(const double* __restrict__ T,
                                                          const double* __restrict__ cond,
@@ -634,7 +634,7 @@ __global__ __launch_bounds__(kThreads) void k_rhs_energy(const double* __restric
         const double djac = djn;
         __syncthreads();
         ring.fetch(min(kk + 2, k1));  // in flight during this step's arithmetic
-        djn = divjac[g.at(i, j, min(kk + 1, k1 - 1))];
+        djn = stream_load<NT>(divjac + g.at(i, j, min(kk + 1, k1 - 1)));
         const int sm = ring_slot(kk - 1), s0 = ring_slot(kk), sp = ring_slot(kk + 1);
         auto slot = [&](int dk) { return dk < 0 ? sm : (dk > 0 ? sp : s0); };
         auto t = [&](int di, int dj, int dk) { return sF[0][slot(dk)][e0 + di + dj * kRingX]; };

@@ -11,6 +11,7 @@
 
 #include <cmath>
 #include <cstdint>
+#include <type_traits>
 #include <vector>
 
 #include "common.h"
@@ -332,6 +333,100 @@ __global__ void k_update_varprop(const double* __restrict__ P, double* U, double
     }
 }
 
+// The variable-density correction reads P, P_now, P_old and rho at the point and
+// at (-1, 0, 0), (0, -1, 0), (0, 0, -1).  A workgroup owns a 64 x 4 tile and
+// marches through a run of planes: a thread loads its own point's values a plane
+// ahead, keeps those of the plane below in registers and hands them to its x
+// and z neighbours through LDS (two slots, one barrier a plane); wave w loads
+// the halo row j0 - 1 of field w and every wave the four fields of its row's
+// x - 1 point.  That is 12 vector memory instructions a point against 22 when
+// every thread read its neighbours itself, which kept the address units 85% busy:
+// at 384x192x256 345 -> 327 us (5.3 TB/s over 67 + 25 B/pt).  On grids that get
+// shorter runs than 16 planes a point per thread is faster, whose loads are all in
+// flight at once (96x48x65: 7.9 against 9.0 us).
+// Loads are unconditional, as PlaneRing's.
+__global__ __launch_bounds__(kTileX * kTileZ) void k_update_varprop_march(
+    const double* __restrict__ P, double* U, double* V, double* W, const double* Uh, const double* Vh,
+    const double* Wh, const double* __restrict__ Pn, const double* __restrict__ Po, const double* __restrict__ rho,
+    const double* __restrict__ hi, const double* __restrict__ lo, const double* __restrict__ rho_min_p, Halo h,
+    BandGrid bg, int kmin_Vhat, double dtmax, double inv_dx, double inv_dz) {
+#pragma clang fp contract(off)
+    constexpr int X = kTileX + 1;  // point (i, j) of the tile at (j + 1) * X + i + 1
+    __shared__ double sF[4][2][X * (kTileZ + 1)];
+    int i0, j0, k0, k1;
+    if (!ring_tile(bg, h.ny, i0, j0, k0, k1)) return;
+    const long sy = h.sy(), sp = (long)h.nx * h.nz;
+    const int row = tile_row(), j = j0 + row;
+    // lanes past the last column repeat its point (same loads, same stores)
+    const int i = min(i0 + (int)threadIdx.x, h.nx - 1);
+    const int x = i - i0 + 1;
+    // field q at (ii, jj) and a plane apart; P has no halo and wraps
+    auto column = [&](int q, int ii, int jj) -> const double* {
+        return q == 0 ? P + pidx(h, ii, jj, 0) : (q == 1 ? Pn : (q == 2 ? Po : rho)) + h.at(ii, jj, 0);
+    };
+    const double* zrow = column(row, i, j0 - 1);
+    const long zs = row == 0 ? sp : sy;
+    if (j >= h.nz) {  // a wave without a row: the halo row of its field
+        for (int k = k0; k < k1; ++k) {
+            sF[row][k & 1][x] = zrow[k * zs];
+            __syncthreads();
+        }
+        return;
+    }
+    const int xq = min((int)threadIdx.x, 3);
+    const double* xcol = column(xq, i0 - 1, j);
+    const long xs = xq == 0 ? sp : sy;
+    struct Ahead {
+        double f[4], z, x, u, v, w;
+    };
+    auto load = [&](int k) {
+        const long c = h.at(i, j, k);
+        return Ahead{{P[pidx(h, i, j, k)], Pn[c], Po[c], rho[c]}, zrow[k * zs], xcol[k * xs], Uh[c], Vh[c], Wh[c]};
+    };
+    const double inv_rho_min = 1.0 / uniform_load(rho_min_p, 0);
+    // the plane below
+    const long cm = h.at(i, j, k0 - 1);
+    double pm = P[pidx(h, i, j, k0 - 1)], psm = 2 * Pn[cm] - Po[cm], rm = rho[cm];
+    Ahead buf[2];
+    buf[0] = load(k0);
+    auto step = [&](auto B, int k) {
+#pragma clang fp contract(off)
+        const Ahead& a = buf[B];
+        const int slot = k & 1, e = (row + 1) * X + x;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) sF[q][slot][e] = a.f[q];
+        sF[row][slot][x] = a.z;
+        sF[xq][slot][(row + 1) * X] = a.x;
+        __syncthreads();
+        buf[B ^ 1] = load(min(k + 1, k1 - 1));
+        const double p = a.f[0], ps_c = 2 * a.f[1] - a.f[2], rc = a.f[3];
+        auto flux = [&](double pb, double ps_b, double rb) {
+            const double inv_rho_now = 0.5 / rc + 0.5 / rb;
+            const double P_fwd = p * inv_rho_min + (inv_rho_now - inv_rho_min) * ps_c;
+            const double P_bwd = pb * inv_rho_min + (inv_rho_now - inv_rho_min) * ps_b;
+            return make_double2(P_fwd, P_bwd);
+        };
+        auto at = [&](int n) { return flux(sF[0][slot][n], 2 * sF[1][slot][n] - sF[2][slot][n], sF[3][slot][n]); };
+        const long c = h.at(i, j, k);
+        double2 f = at(e - 1);
+        U[c] = a.u - dtmax * (f.x - f.y) * inv_dx;
+        f = at(e - X);
+        W[c] = a.w - dtmax * (f.x - f.y) * inv_dz;
+        f = flux(pm, psm, rm);
+        const double v = a.v - dtmax * (uniform_load(hi, k) * f.x + uniform_load(lo, k) * f.y);
+        if (k >= kmin_Vhat) V[c] = v;
+        pm = p;
+        psm = ps_c;
+        rm = rc;
+    };
+    for (int k = k0;;) {
+        step(std::integral_constant<int, 0>(), k);
+        if (++k >= k1) break;
+        step(std::integral_constant<int, 1>(), k);
+        if (++k >= k1) break;
+    }
+}
+
 // P_per over the whole padded array, and (varprop) P_old <- P_now, P_now <- P_per
 // One thread per padded point, x fastest (a pure stream: no tiles, so no
 // idle lanes on the nx + 2 wide rows); IDX32: the padded array has fewer
@@ -478,10 +573,14 @@ int update_vars_interior(const double* P, double* P_per, double* P_now, double* 
                          int kmin_Vhat, double dtmax, double inv_dx, double inv_dz, int use_incompressible,
                          hipStream_t st) {
     const Halo h{nx, nz, ny};
-    const BandGrid bg = band_grid(nx, nz, ny);
+    const BandGrid bg = band_grid(nx, nz, ny), br = ring_grid(nx, nz, ny);
     if (use_incompressible)
         k_update_incomp<<<bg.blocks(), band_block(), 0, st>>>(P, U, V, W, U_hat, V_hat, W_hat, hi, lo, h, bg,
                                                               kmin_Vhat, dtmax, inv_dx, inv_dz);
+    else if (br.run == kRunK)
+        k_update_varprop_march<<<br.blocks(), band_block(), 0, st>>>(P, U, V, W, U_hat, V_hat, W_hat, P_now, P_old, rho,
+                                                                     hi, lo, rho_min, h, br, kmin_Vhat, dtmax, inv_dx,
+                                                                     inv_dz);
     else
         k_update_varprop<<<bg.blocks(), band_block(), 0, st>>>(P, U, V, W, U_hat, V_hat, W_hat, P_now, P_old, rho, hi,
                                                                lo, rho_min, h, bg, kmin_Vhat, dtmax, inv_dx, inv_dz);
