@@ -259,7 +259,7 @@ __global__ __launch_bounds__(kThreads) void k_momentum(
     }
     const int i = min(i0 + (int)threadIdx.x, g.nx - 1);
     const int e0 = (row + 1) * kRingX + (i - i0) + 1;
-    const long sz = g.sz(), sy = g.sy();
+    const long sz = g.sz();
     // this point's rho, div_now and buoy with their x and z neighbours, and the
     // last step's R: loaded a plane ahead
     struct Ahead {
