@@ -524,9 +524,20 @@ int dnsp_poisson_get_variants(const dnsp_poisson* h, int* xvar, int* zvar, int* 
     return DNSP_OK;
 }
 
+// Values in (-1, 1) for the tuner's timed launches.  On zeros the kernels draw less
+// power and the order of two variants can change: at 768x384x384 the two-pass
+// tridiagonal was picked, 375-380 us inside a solve, over the one-pass one's 365.
+static __global__ __launch_bounds__(256) void k_tune_fill(double* __restrict__ a, long n) {
+    for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
+        unsigned long long z = (unsigned long long)i * 0x9E3779B97F4A7C15ull;
+        z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+        a[i] = (double)(long long)(z ^ (z >> 27)) * 0x1p-63;
+    }
+}
+
 // Times each FFT kernel variant per direction (`reps` forward transforms,
 // then `reps` inverse ones, keeping the fastest of each) and pairs of
-// tridiagonal solves per partitioned variant, on `work` (zero-filled first;
+// tridiagonal solves per partitioned variant, on `work` (filled first;
 // NULL = a temporary device array); for a mixed-precision handle the same
 // for its kernels.  times_ms (optional, DNSP_TUNE_SLOTS entries): mean ms of
 // a forward + inverse pair of the x, z (4 slots each) and of a pair of
@@ -566,10 +577,10 @@ int dnsp_poisson_autotune(dnsp_poisson* h, double* work, int reps, void* stream,
         *per = (double)ms / n;
         return DNSP_OK;
     };
+    auto fill = [&]() { k_tune_fill<<<2048, 256, 0, st>>>(buf, (long)N); };
     do {
-        if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess ||
-            hipMemsetAsync(buf, 0, sizeof(double) * N, st) != hipSuccess) {
-            set_error("autotune: event or memset failed");
+        if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
+            set_error("autotune: event creation failed");
             rc = DNSP_ERR_HIP;
             break;
         }
@@ -583,6 +594,7 @@ int dnsp_poisson_autotune(dnsp_poisson* h, double* work, int reps, void* stream,
             for (int v = 0; v < nvar && rc == DNSP_OK; ++v) {
                 *knob[kf] = v;
                 *knob[kb] = v;
+                fill();  // repeated transforms scale the values
                 rc = dnsp_poisson_stage(h, buf, buf, sf, stream);  // warm-up
                 if (!rc) rc = dnsp_poisson_stage(h, buf, buf, sb, stream);
                 double tf = 0.0, tb = 0.0;
@@ -603,12 +615,9 @@ int dnsp_poisson_autotune(dnsp_poisson* h, double* work, int reps, void* stream,
         }
         if (rc || !h->blk_ok) break;
         // the blocked solve's own knobs, timed stage by stage through
-        // dnsp_poisson_solve_stage on buf (rhs and solution) and the workspace
-        if (hipMemsetAsync(h->d_W, 0, sizeof(double) * N, st) != hipSuccess) {
-            set_error("autotune: memset failed");
-            rc = DNSP_ERR_HIP;
-            break;
-        }
+        // dnsp_poisson_solve_stage on buf (rhs and solution) and the workspace; a
+        // stage leaves its input in place (the last one's scaled by each pass)
+        fill();
         const bool on = h->blk_on;
         h->blk_on = true;
         auto timed_b = [&](int stage, double* per) -> int {
