@@ -465,7 +465,11 @@ static int poisson_apply_strategy(dnsp_poisson* h) {
     h->blk_ok = rg && rg_supported(h->nx) && rg_supported(h->nz) && h->nx % 16 == 0 && part;
     if (h->blk_ok && !h->d_W) {
         const size_t N = (size_t)h->nx * h->nz * h->ny;
-        DNSP_HIP_TRY(hipMalloc(&h->d_W, sizeof(double) * N));
+        if (hipMalloc(&h->d_W, sizeof(double) * N) != hipSuccess) {  // the in-place stages need none
+            (void)hipGetLastError();
+            h->d_W = nullptr;
+            h->blk_ok = false;
+        }
     }
     return DNSP_OK;
 }
