@@ -581,6 +581,9 @@ int dnsp_poisson_autotune(dnsp_poisson* h, double* work, int reps, void* stream,
         *per = (double)ms / n;
         return DNSP_OK;
     };
+    // a register-direct handle with a blocked solve: the tridiagonal variants are
+    // timed once, in the blocked layouts that its solves use
+    const bool tri_blk = h->blk_ok && (h->rx || h->rz);
     auto fill = [&]() { k_tune_fill<<<2048, 256, 0, st>>>(buf, (long)N); };
     do {
         if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
@@ -590,7 +593,7 @@ int dnsp_poisson_autotune(dnsp_poisson* h, double* work, int reps, void* stream,
         }
         for (int dir = 0; dir < 3 && rc == DNSP_OK; ++dir) {
             const bool has = dir == 0 ? h->ct_x : dir == 1 ? h->ct_z : h->part_rows > 0;
-            if (!has) continue;
+            if (!has || (dir == 2 && tri_blk)) continue;
             const int nvar = dir == 2 ? kPartVariants : kCtVariants;
             const int sf = dir == 0 ? DNSP_STAGE_X_FWD : dir == 1 ? DNSP_STAGE_Z_FWD : DNSP_STAGE_TRIDIAG;
             const int sb = dir == 0 ? DNSP_STAGE_X_BWD : dir == 1 ? DNSP_STAGE_Z_BWD : DNSP_STAGE_TRIDIAG;
@@ -643,18 +646,25 @@ int dnsp_poisson_autotune(dnsp_poisson* h, double* work, int reps, void* stream,
         const int nx_v = h->rx ? 1 : kCtVariants, nz_v = h->rz ? 1 : 2;  // register-direct: one shape
         const int nv[5] = {nx_v, nz_v, kPartVariants, nz_v, nx_v};
         for (int stage = 0; stage < 5 && !rc; ++stage) {
+            if (nv[stage] == 1) {  // nothing to choose: only fill what the next stage reads
+                *bk[stage] = 0;
+                rc = dnsp_poisson_solve_stage(h, buf, buf, stage, stream);
+                continue;
+            }
             double bt = 1e30;
             int bv = *bk[stage];
             for (int v = 0; v < nv[stage] && !rc; ++v) {
                 *bk[stage] = v;
                 double t = 0.0;
                 rc = timed_b(stage, &t);
+                if (!rc && stage == 2 && tri_blk && times_ms) times_ms[kTuneSlot[2] + v] = 2.0 * t;
                 if (!rc && t < bt) {
                     bt = t;
                     bv = v;
                 }
             }
             *bk[stage] = bv;
+            if (stage == 2 && tri_blk) pick[4] = bv;
         }
         h->blk_on = on;
     } while (0);
