@@ -856,22 +856,26 @@ int upload_inst(dnsp_batch* b) {
     return DNSP_OK;
 }
 
-// One instance through the blocked stages (dnsp_poisson_solve_stage).
-void run_alone(const BInst& I, double* W, hipStream_t st) {
+// One instance through the blocked stages (dnsp_poisson_solve_stage).  d: its
+// entry of the device table, whose f and P the kernels read when they run, as
+// those of the shared launches do: a captured run follows a later bind.
+void run_alone(const BInst& I, BInst* d, double* W, hipStream_t st) {
     const size_t N = (size_t)I.plane * (size_t)I.ny;
-    xb_x_launch(I.nx, blk_xfwd_variant(N), I.f, W, I.nlines, I.nz, I.twx, st);
-    mm_z_launch(I.nz, kBlkZVariant, false, W, I.P, I.nx, I.ny, I.twz, st);
-    part_launch<double, double, true>(kPartDefault, I.P, I.ax, I.az, I.bands, I.nx, I.nz, I.ny, I.pcr_min, nullptr,
-                                      nullptr, 0.0, st, nullptr, 0, W);
-    mm_z_launch(I.nz, kBlkZVariant, true, W, I.P, I.nx, I.ny, I.twz, st);
-    ct_x_launch(I.nx, blk_xbwd_variant(I.nx), true, I.P, I.P, I.nlines, I.twx, I.inv_nxnz, st);
+    xb_x_launch(I.nx, blk_xfwd_variant(N), nullptr, W, I.nlines, I.nz, I.twx, st, &d->f);
+    mm_z_launch(I.nz, kBlkZVariant, false, W, nullptr, I.nx, I.ny, I.twz, st, &d->P);
+    static_assert(kPartDefault == 2, "one-pass rule-shaped tridiagonal");
+    PartArgs<double> t{nullptr, I.ax, I.az, I.bands, I.nx, I.nz, I.ny, I.pcr_min, nullptr, nullptr, 0.0, nullptr, 0, W,
+                       &d->P};
+    part_launch_rule<double, double, false, true>(t, st);
+    mm_z_launch(I.nz, kBlkZVariant, true, W, nullptr, I.nx, I.ny, I.twz, st, &d->P);
+    ct_x_launch(I.nx, blk_xbwd_variant(I.nx), true, nullptr, nullptr, I.nlines, I.twx, I.inv_nxnz, st, &d->P);
 }
 
 void run_fp64(dnsp_batch* b, int xv, int zv, int tv, hipStream_t st) {
     const bool split = tv == 6 && !b->alone.empty();
     if (tv == 6) tv = 4;
     if (split)
-        for (int i : b->alone) run_alone(b->h_inst[(size_t)i], b->d_W, st);
+        for (int i : b->alone) run_alone(b->h_inst[(size_t)i], b->d_inst + i, b->d_W, st);
     const std::vector<BGroup>&gx = split ? b->sx[xv] : b->gx[xv], &gz = split ? b->sz[zv] : b->gz[zv],
                             &gt = split ? b->st : b->gt;
     for (const BGroup& g : gx) bx_launch(BX_F64_FWD, xv, b->d_inst, g, 0, st);

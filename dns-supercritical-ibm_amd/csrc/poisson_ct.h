@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <climits>
+#include <cstdint>
 
 #include "fft_ct.h"
 
@@ -27,6 +28,15 @@ __device__ __forceinline__ double2 stream_load(const double2* p) {
     } else {
         return *p;
     }
+}
+// The array of a kernel of the blocked solve: p, or (at not NULL) the one whose
+// address stands at `at` when the kernel runs.  A batch passes the places in its
+// instance table, so that a captured launch follows a later bind.
+template <typename T>
+__device__ __forceinline__ T* array_at(T* p, T* const* at) {
+    typedef T __attribute__((address_space(1))) * GlobalPtr;
+    // by its integer value: a pointer read from memory would be a flat one
+    return (T*)(GlobalPtr)(at ? *reinterpret_cast<const uintptr_t*>(at) : reinterpret_cast<uintptr_t>(p));
 }
 // The z transforms of 512 points keep ordinary loads: 384x512x256 takes 846 us with
 // them, 874 past the caches (z forward alone at 512x512x288 267 and 305).
@@ -261,11 +271,11 @@ __device__ __forceinline__ void xbwd_body(const double* S, double* P, long nline
 
 template <int N, int G, int NT>
 __global__ __launch_bounds__(NT) void kt_xbwd(const double* S, double* P, long nlines,
-                                              const double2* __restrict__ tw, double scale) {
+                                              const double2* __restrict__ tw, double scale, double* const* at) {
     __shared__ double2 sm[G * ct_pitch(N)];
     __shared__ double2 stw[N];
     ct_stage_twiddles<N, NT>(stw, tw);
-    xbwd_body<N, G, NT>(S, P, nlines, stw, scale, xcd_tile(blockIdx.x, gridDim.x), sm);
+    xbwd_body<N, G, NT>(array_at<const double>(S, at), array_at(P, at), nlines, stw, scale, xcd_tile(blockIdx.x, gridDim.x), sm);
 }
 
 // ---------------------------------------------------------------------------
@@ -525,24 +535,25 @@ __host__ __device__ constexpr int lds_waves(int lds, int nt, int cap = 8) {
 }
 template <int N, int G, int NT>
 __global__ __launch_bounds__(NT) void kt_xfwd_xb(const double* P, double* W, long nlines, int nz,
-                                                 const double2* __restrict__ tw) {
+                                                 const double2* __restrict__ tw, const double* const* at) {
     __shared__ double2 sm[G * ct_pitch(N)];
     __shared__ double2 stw[N];
     ct_stage_twiddles<N, NT>(stw, tw);
-    xfwd_body<N, G, NT, true>(P, W, nlines, stw, xcd_tile(blockIdx.x, gridDim.x), sm, nz);
+    xfwd_body<N, G, NT, true>(array_at(P, at), W, nlines, stw, xcd_tile(blockIdx.x, gridDim.x), sm, nz);
 }
 
 // z forward, XB -> MM.  Tile (k, c): the 16 x rows 16c..16c+15 of plane k as
 // 8 complex columns (rows 2t and 2t + 1 paired as in kt_zfwd); N = nz.
 template <int N, int NT>
 __global__ __launch_bounds__(NT) void kt_zfwd_mm(const double* __restrict__ W, double* __restrict__ S, int nx,
-                                                 int ny, const double2* __restrict__ tw) {
+                                                 int ny, const double2* __restrict__ tw, double* const* at) {
     constexpr int TA = 8;
     constexpr int LP = ct_pitch(N);
     constexpr int TOT2 = TA * N;
     constexpr int NL2 = (TOT2 + NT - 1) / NT;
     __shared__ double2 sm[TA * LP];
     __shared__ double2 stw[N];
+    double* const D = array_at<double>(S, at);
     ct_stage_twiddles<N, NT>(stw, tw);
     const int nab = nx / 16;
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
@@ -563,7 +574,7 @@ __global__ __launch_bounds__(NT) void kt_zfwd_mm(const double* __restrict__ W, d
     }
     __syncthreads();
     fft_ct<N, TA, NT, false>(sm, stw);
-    double* dst = S + (size_t)c * N * ny * 16 + (size_t)k * 16;
+    double* dst = D + (size_t)c * N * ny * 16 + (size_t)k * 16;
 #pragma unroll
     for (int q = 0; q < NL2; ++q) {
         const int e = (int)threadIdx.x + q * NT;
@@ -585,7 +596,7 @@ __global__ __launch_bounds__(NT) void kt_zfwd_mm(const double* __restrict__ W, d
 // kt_zbwd from the tile's contiguous block of W; N = nz.
 template <int N, int NT>
 __global__ __launch_bounds__(NT) void kt_zbwd_xl(const double* __restrict__ W, double* __restrict__ P, int nx,
-                                                 int ny, const double2* __restrict__ tw) {
+                                                 int ny, const double2* __restrict__ tw, double* const* at) {
     constexpr int TA = 8;
     constexpr int LP = ct_pitch(N);
     constexpr int H = N / 2 + 1;
@@ -594,6 +605,7 @@ __global__ __launch_bounds__(NT) void kt_zbwd_xl(const double* __restrict__ W, d
     constexpr int NL2 = (TOT2 + NT - 1) / NT;
     __shared__ double2 sm[TA * LP];
     __shared__ double2 stw[N];
+    double* const D = array_at<double>(P, at);
     ct_stage_twiddles<N, NT>(stw, tw);
     const int nab = nx / 16;
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
@@ -626,7 +638,7 @@ __global__ __launch_bounds__(NT) void kt_zbwd_xl(const double* __restrict__ W, d
     }
     __syncthreads();
     fft_ct<N, TA, NT, true>(sm, stw);
-    double* dst = P + (size_t)k * nx * N + (size_t)c * 16;
+    double* dst = D + (size_t)k * nx * N + (size_t)c * 16;
 #pragma unroll
     for (int q = 0; q < NL2; ++q) {
         const int e = (int)threadIdx.x + q * NT;
@@ -1071,7 +1083,7 @@ __global__ __launch_bounds__(M * P, OCC) void kt_tri_part(T* S, const double* __
                                                           double* __restrict__ pbar = nullptr,
                                                           double inv_nxnz = 0.0,
                                                           const int* __restrict__ glist = nullptr, int nz = 0,
-                                                          T* So = nullptr) {
+                                                          T* So = nullptr, T* const* at = nullptr) {
     __shared__ TriRed<P, M, Ar> red;
     extern __shared__ double smb_raw[];  // the group's band set, 3 * MR * P values
     Ar* smb = reinterpret_cast<Ar*>(smb_raw);
@@ -1090,6 +1102,7 @@ __global__ __launch_bounds__(M * P, OCC) void kt_tri_part(T* S, const double* __
             mode = g16 < 0 ? LONG_MAX : tri_group_mode(g16, (plane + 15) / 16, 16, mi % 16);
         }
     }
+    if constexpr (MM) S = array_at(S, at);
     Ar d[MR];
     const double lam64 = tri_prologue<MR, P, M, T, Ar, MM>(d, smb, bands + (grp == 0 ? 3 * ny : 0), S, ax, az, mode,
                                                            plane, nx, ny, msum, nz);

@@ -9,17 +9,20 @@
 namespace dnsp {
 
 bool ct_fft_supported(int n);
+// at (inverse only; device, NULL: src and dst): the place of the address of the
+// array to transform in place, read when the kernel runs (array_at).
 void ct_x_launch(int n, int variant, bool inv, const double* src, double* dst, long nlines, const double2* tw,
-                 double scale, hipStream_t st);
+                 double scale, hipStream_t st, double* const* at = nullptr);
 void ct_z_launch(int n, int variant, bool inv, double* S, int nx, int ny, const double2* tw, hipStream_t st);
 // The blocked FP64 solve (poisson_ct.h): the x forward transform from lines
 // to the x-blocked layout (variants as ct_x_launch); the z transforms from
 // x-blocked to mode-major (forward) and from x-blocked to halfcomplex lines
-// (inverse), variant 0: 256 threads, 1: 512.
+// (inverse), variant 0: 256 threads, 1: 512.  at: the place of the address of
+// the caller's array (src of xb_x_launch, dst of mm_z_launch), as ct_x_launch.
 void xb_x_launch(int n, int variant, const double* src, double* dst, long nlines, int nz, const double2* tw,
-                 hipStream_t st);
+                 hipStream_t st, const double* const* at = nullptr);
 void mm_z_launch(int n, int variant, bool inv, const double* src, double* dst, int nx, int ny, const double2* tw,
-                 hipStream_t st);
+                 hipStream_t st, double* const* at = nullptr);
 // The FP64 transforms of every length 16..768 with prime factors up to 13
 // (poisson_reg.h; strides and layouts there).  z: mm = 1 writes the
 // mode-major blocks, 0 back in place.
@@ -115,6 +118,7 @@ struct PartArgs {
     const int* glist;
     int nlist;
     T* So;
+    T* const* at = nullptr;  // MM: the place of S's address, as ct_x_launch
 };
 template <typename T, typename Ar, bool TP, bool MM>
 void part_launch_rule(const PartArgs<T>& a, hipStream_t st);

@@ -31,19 +31,20 @@ static void ct_z_v(int v, bool inv, T* S, int nx, int ny, const typename Cx<T>::
 }
 
 template <int N, int NT>
-static void mm_z(bool inv, const double* src, double* dst, int nx, int ny, const double2* tw, hipStream_t st) {
+static void mm_z(bool inv, const double* src, double* dst, int nx, int ny, const double2* tw, hipStream_t st,
+                 double* const* at) {
     const int nb = (nx / 16) * ny;
-    if (!inv) kt_zfwd_mm<N, NT><<<nb, NT, 0, st>>>(src, dst, nx, ny, tw);
-    else      kt_zbwd_xl<N, NT><<<nb, NT, 0, st>>>(src, dst, nx, ny, tw);
+    if (!inv) kt_zfwd_mm<N, NT><<<nb, NT, 0, st>>>(src, dst, nx, ny, tw, at);
+    else      kt_zbwd_xl<N, NT><<<nb, NT, 0, st>>>(src, dst, nx, ny, tw, at);
 }
 
 void mm_z_launch(int n, int variant, bool inv, const double* src, double* dst, int nx, int ny, const double2* tw,
-                 hipStream_t st) {
+                 hipStream_t st, double* const* at) {
     switch (n) {
 #define DNSP_CASE(N)                                                     \
     case N:                                                              \
-        if (variant == 0) mm_z<N, 256>(inv, src, dst, nx, ny, tw, st);   \
-        else mm_z<N, 512>(inv, src, dst, nx, ny, tw, st);                \
+        if (variant == 0) mm_z<N, 256>(inv, src, dst, nx, ny, tw, st, at); \
+        else mm_z<N, 512>(inv, src, dst, nx, ny, tw, st, at);            \
         break;
         DNSP_CT_SIZES(DNSP_CASE)
 #undef DNSP_CASE

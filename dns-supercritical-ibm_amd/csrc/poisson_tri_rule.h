@@ -18,7 +18,7 @@ void rule_launch(const PartArgs<T>& a, hipStream_t st) {
     const int ngroups = a.glist ? a.nlist / (M == 32 ? 2 : 1) : (int)((plane + M - 1) / M) + 1;
     if (ngroups <= 0) return;
     kt_tri_part<MR, P, M, T, 1, TP, Ar, MM><<<ngroups, M * P, 3 * sizeof(Ar) * MR * P, st>>>(
-        a.S, a.ax, a.az, a.bands, a.nx, a.ny, plane, a.pcr_min, a.msum, a.pbar, a.inv_nxnz, a.glist, a.nz, a.So);
+        a.S, a.ax, a.az, a.bands, a.nx, a.ny, plane, a.pcr_min, a.msum, a.pbar, a.inv_nxnz, a.glist, a.nz, a.So, a.at);
 }
 
 // chunk counts and their row ranges, from part_shape's bounds
