@@ -457,19 +457,20 @@ static int poisson_apply_strategy(dnsp_poisson* h) {
         const size_t N = (size_t)h->nx * h->nz * h->ny;
         DNSP_HIP_TRY(hipMalloc(&h->d_cp, sizeof(double) * N));
     }
-    // the blocked solve: compile-time or register-direct x and z transforms,
-    // nx a multiple of 16, the partitioned tridiagonal; its workspace is one field
     const bool rg = h->fft_strategy == DNSP_FFT_AUTO;
     h->rx = rg && !h->ct_x ? rg_ops(h->nx) : nullptr;
     h->rz = rg && !h->ct_z ? rg_ops(h->nz) : nullptr;
-    h->blk_ok = rg && rg_supported(h->nx) && rg_supported(h->nz) && h->nx % 16 == 0 && part;
+    // the blocked solve: compile-time x and z transforms (all their lengths are
+    // multiples of 16), the partitioned tridiagonal; its workspace is one field.
+    // Not with register-direct transforms: a handle of such lengths writes the
+    // caller's array only, so that solves of several streams on it may overlap, and
+    // the in-place stages are as fast (us per solve, in place / blocked: 336x210x200
+    // 191 / 200, 560x280x280 721 / 722, 624x312x770 2528 / 2526, 720x360x360 1551 / 1512,
+    // 512x280x200 386 / 448, 560x256x300 697 / 670).
+    h->blk_ok = rg && h->ct_x && h->ct_z && part;
     if (h->blk_ok && !h->d_W) {
         const size_t N = (size_t)h->nx * h->nz * h->ny;
-        if (hipMalloc(&h->d_W, sizeof(double) * N) != hipSuccess) {  // the in-place stages need none
-            (void)hipGetLastError();
-            h->d_W = nullptr;
-            h->blk_ok = false;
-        }
+        DNSP_HIP_TRY(hipMalloc(&h->d_W, sizeof(double) * N));
     }
     return DNSP_OK;
 }
@@ -581,9 +582,6 @@ int dnsp_poisson_autotune(dnsp_poisson* h, double* work, int reps, void* stream,
         *per = (double)ms / n;
         return DNSP_OK;
     };
-    // a register-direct handle with a blocked solve: the tridiagonal variants are
-    // timed once, in the blocked layouts that its solves use
-    const bool tri_blk = h->blk_ok && (h->rx || h->rz);
     auto fill = [&]() { k_tune_fill<<<2048, 256, 0, st>>>(buf, (long)N); };
     do {
         if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
@@ -593,7 +591,7 @@ int dnsp_poisson_autotune(dnsp_poisson* h, double* work, int reps, void* stream,
         }
         for (int dir = 0; dir < 3 && rc == DNSP_OK; ++dir) {
             const bool has = dir == 0 ? h->ct_x : dir == 1 ? h->ct_z : h->part_rows > 0;
-            if (!has || (dir == 2 && tri_blk)) continue;
+            if (!has) continue;
             const int nvar = dir == 2 ? kPartVariants : kCtVariants;
             const int sf = dir == 0 ? DNSP_STAGE_X_FWD : dir == 1 ? DNSP_STAGE_Z_FWD : DNSP_STAGE_TRIDIAG;
             const int sb = dir == 0 ? DNSP_STAGE_X_BWD : dir == 1 ? DNSP_STAGE_Z_BWD : DNSP_STAGE_TRIDIAG;
@@ -643,28 +641,20 @@ int dnsp_poisson_autotune(dnsp_poisson* h, double* work, int reps, void* stream,
             return DNSP_OK;
         };
         int* bk[5] = {&h->bxvar, &h->bzvar, &h->btvar, &h->bzvar_b, &h->bxvar_b};  // by stage
-        const int nx_v = h->rx ? 1 : kCtVariants, nz_v = h->rz ? 1 : 2;  // register-direct: one shape
-        const int nv[5] = {nx_v, nz_v, kPartVariants, nz_v, nx_v};
+        const int nv[5] = {kCtVariants, 2, kPartVariants, 2, kCtVariants};
         for (int stage = 0; stage < 5 && !rc; ++stage) {
-            if (nv[stage] == 1) {  // nothing to choose: only fill what the next stage reads
-                *bk[stage] = 0;
-                rc = dnsp_poisson_solve_stage(h, buf, buf, stage, stream);
-                continue;
-            }
             double bt = 1e30;
             int bv = *bk[stage];
             for (int v = 0; v < nv[stage] && !rc; ++v) {
                 *bk[stage] = v;
                 double t = 0.0;
                 rc = timed_b(stage, &t);
-                if (!rc && stage == 2 && tri_blk && times_ms) times_ms[kTuneSlot[2] + v] = 2.0 * t;
                 if (!rc && t < bt) {
                     bt = t;
                     bv = v;
                 }
             }
             *bk[stage] = bv;
-            if (stage == 2 && tri_blk) pick[4] = bv;
         }
         h->blk_on = on;
     } while (0);
@@ -820,30 +810,18 @@ int dnsp_poisson_solve_stage(dnsp_poisson* h, const double* rhs, double* P, int 
         return dnsp_poisson_stage(h, stage == 0 ? rhs : P, P, st_of[stage], stream);
     }
     hipStream_t st = as_stream(stream);
-    const long nlines = (long)h->nz * h->ny, plane = (long)h->nx * h->nz;
+    const long nlines = (long)h->nz * h->ny;
     const double inv_nxnz = 1.0 / ((double)h->nx * (double)h->nz + 0.0);
     // P lines -> W x-blocked -> P mode-major -> W x-blocked -> P lines -> P
     switch (stage) {
-        case 0:
-            if (h->rx) h->rx->xfwd(rhs, h->d_W, nlines, h->nz, plane, 16, h->nz * 16, h->d_twx, st);
-            else xb_x_launch(h->nx, h->bxvar, rhs, h->d_W, nlines, h->nz, h->d_twx, st);
-            break;
-        case 1:
-            if (h->rz) h->rz->zfwd(h->d_W, P, h->nx, h->ny, plane, h->nz * 16, 16, 1, h->d_twz, st);
-            else mm_z_launch(h->nz, h->bzvar, false, h->d_W, P, h->nx, h->ny, h->d_twz, st);
-            break;
+        case 0: xb_x_launch(h->nx, h->bxvar, rhs, h->d_W, nlines, h->nz, h->d_twx, st); break;
+        case 1: mm_z_launch(h->nz, h->bzvar, false, h->d_W, P, h->nx, h->ny, h->d_twz, st); break;
         case 2:
             part_launch<double, double, true>(h->btvar, P, h->d_ax, h->d_az, h->d_bands, h->nx, h->nz, h->ny,
                                               h->pcr_min, nullptr, nullptr, 0.0, st, nullptr, 0, h->d_W);
             break;
-        case 3:
-            if (h->rz) h->rz->zbwd(h->d_W, P, h->nx, h->ny, plane, h->nz * 16, 16, h->d_twz, st);
-            else mm_z_launch(h->nz, h->bzvar_b, true, h->d_W, P, h->nx, h->ny, h->d_twz, st);
-            break;
-        default:
-            if (h->rx) h->rx->xbwd(P, P, nlines, inv_nxnz, h->d_twx, st);
-            else ct_x_launch(h->nx, h->bxvar_b, true, P, P, nlines, h->d_twx, inv_nxnz, st);
-            break;
+        case 3: mm_z_launch(h->nz, h->bzvar_b, true, h->d_W, P, h->nx, h->ny, h->d_twz, st); break;
+        default: ct_x_launch(h->nx, h->bxvar_b, true, P, P, nlines, h->d_twx, inv_nxnz, st); break;
     }
     DNSP_LAUNCH_CHECK();
     return DNSP_OK;

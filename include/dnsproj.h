@@ -117,18 +117,19 @@ int dnsp_poisson_solve_stage(dnsp_poisson* h, const double* rhs, double* P, int 
 
 /* Blocked solve (no counterpart in the reference; same arithmetic, results
  * bit-identical to the in-place stages with the same kernel variants): for
- * nx a multiple of 16, x and z lengths of 16..768 with prime factors up to 13,
- * and the partitioned tridiagonal, dnsp_poisson_run / dnsp_poisson_solve go through a workspace
+ * nx a multiple of 16 with the compile-time FFT kernels and the partitioned
+ * tridiagonal, dnsp_poisson_run / dnsp_poisson_solve go through a workspace
  * of one field held by the handle: x-transformed lines go to an x-blocked
  * layout [k][a/16][j][a%16], the z transform turns that into mode-major
  * blocks [a/16][b][k][a%16], the tridiagonal solve writes the x-blocked
  * layout back, the inverse z transform halfcomplex lines, so that every z
  * tile and tridiagonal mode group reads a contiguous block of memory.  On (1) by default where supported;
  * dnsp_poisson_set_blocked(h, 0) returns to the in-place stages.  Arrays
- * that are not 16-byte aligned take the in-place stages, and so does a handle
- * whose workspace could not be allocated (supported reads 0).  The workspace
+ * that are not 16-byte aligned take the in-place stages.  The workspace
  * makes concurrent solves on one handle race (as the reference's shared work
- * arrays do). */
+ * arrays do); a handle that does not run the blocked solve writes nothing but
+ * the caller's array in its FP64 form (the serial tridiagonal's workspace
+ * apart), so that its solves may overlap. */
 int dnsp_poisson_set_blocked(dnsp_poisson* h, int on);
 int dnsp_poisson_get_blocked(const dnsp_poisson* h, int* supported, int* on);
 /* The variants of the five kernels dnsp_poisson_solve runs now (stage order:
