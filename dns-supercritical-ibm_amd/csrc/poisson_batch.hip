@@ -544,8 +544,8 @@ struct dnsp_batch {
     std::vector<BGroup> gx[kCtVariants], gz[kCtVariants], gt;
     BGroup gq;
     int max_ny = 0;
-    // variant 6: the instances that run alone and their workspace (NULL: none,
-    // or no memory for it, and every instance runs in the shared launches);
+    // variant 6: the instances that run alone and their workspace (NULL: none
+    // yet, or no memory for it, and every instance runs in the shared launches);
     // the launch groups of the others
     std::vector<int> alone;
     double* d_W = nullptr;
@@ -582,6 +582,7 @@ void release(dnsp_batch* b) {
     int cur = 0;
     if (hipGetDevice(&cur) == hipSuccess && cur != b->device) (void)hipSetDevice(b->device);
     for (void* p : b->allocs) (void)hipFree(p);
+    (void)hipFree(b->d_W);
     if (cur != b->device) (void)hipSetDevice(cur);
     delete b;
 }
@@ -751,35 +752,29 @@ int setup_eig(dnsp_batch* b, const double* inv_dx, const double* inv_dz) {
     return DNSP_OK;
 }
 
-// The instances variant 6 runs alone, and their workspace.
-int setup_alone(dnsp_batch* b) {
+size_t points(const BInst& I) { return (size_t)I.plane * (size_t)I.ny; }
+
+// The workspace of the instances that run alone, as large as the largest one;
+// none without memory for it, the shared launches need none.
+void alone_workspace(dnsp_batch* b) {
+    if (b->d_W || b->alone.empty()) return;
     size_t most = 0;
-    for (int i = 0; i < b->n; ++i) {
-        const BInst& I = b->h_inst[(size_t)i];
-        const size_t N = (size_t)I.plane * (size_t)I.ny;
-        if (N < kBatchAlone) continue;
-        b->alone.push_back(i);
-        most = std::max(most, N);
-    }
-    if (!most) return DNSP_OK;
-    void* w = nullptr;
-    if (hipMalloc(&w, sizeof(double) * most) != hipSuccess) {  // the shared launches need none
+    for (int i : b->alone) most = std::max(most, points(b->h_inst[(size_t)i]));
+    int cur = 0;
+    if (hipGetDevice(&cur) == hipSuccess && cur != b->device) (void)hipSetDevice(b->device);
+    if (hipMalloc(&b->d_W, sizeof(double) * most) != hipSuccess) {
         (void)hipGetLastError();
-        b->alone.clear();
-        return DNSP_OK;
+        b->d_W = nullptr;
     }
-    b->allocs.push_back(w);
-    b->d_W = static_cast<double*>(w);
-    return DNSP_OK;
+    if (cur != b->device) (void)hipSetDevice(cur);
 }
 
 int setup_groups(dnsp_batch* b) {
     const int n = b->n;
-    std::vector<char> shared((size_t)n, 1);
-    for (int i : b->alone) shared[(size_t)i] = 0;
+    for (int i = 0; i < n; ++i)
+        if (points(b->h_inst[(size_t)i]) >= kBatchAlone) b->alone.push_back(i);
     auto rest = [&](std::vector<long> t) {  // the tasks of the instances that do not run alone
-        for (int i = 0; i < n; ++i)
-            if (!shared[(size_t)i]) t[(size_t)i] = 0;
+        for (int i : b->alone) t[(size_t)i] = 0;
         return t;
     };
     for (int v = 0; v < kCtVariants; ++v) {
@@ -860,8 +855,7 @@ int upload_inst(dnsp_batch* b) {
 // entry of the device table, whose f and P the kernels read when they run, as
 // those of the shared launches do: a captured run follows a later bind.
 void run_alone(const BInst& I, BInst* d, double* W, hipStream_t st) {
-    const size_t N = (size_t)I.plane * (size_t)I.ny;
-    xb_x_launch(I.nx, blk_xfwd_variant(N), nullptr, W, I.nlines, I.nz, I.twx, st, &d->f);
+    xb_x_launch(I.nx, blk_xfwd_variant(points(I)), nullptr, W, I.nlines, I.nz, I.twx, st, &d->f);
     mm_z_launch(I.nz, kBlkZVariant, false, W, nullptr, I.nx, I.ny, I.twz, st, &d->P);
     static_assert(kPartDefault == 2, "one-pass rule-shaped tridiagonal");
     PartArgs<double> t{nullptr, I.ax, I.az, I.bands, I.nx, I.nz, I.ny, I.pcr_min, nullptr, nullptr, 0.0, nullptr, 0, W,
@@ -872,7 +866,7 @@ void run_alone(const BInst& I, BInst* d, double* W, hipStream_t st) {
 }
 
 void run_fp64(dnsp_batch* b, int xv, int zv, int tv, hipStream_t st) {
-    const bool split = tv == 6 && !b->alone.empty();
+    const bool split = tv == 6 && b->d_W;
     if (tv == 6) tv = 4;
     if (split)
         for (int i : b->alone) run_alone(b->h_inst[(size_t)i], b->d_inst + i, b->d_W, st);
@@ -985,6 +979,7 @@ int dnsp_batch_create(int n, const int* nx, const int* nz, const int* ny, const 
     }
     b->n = n;
     b->precision = precision;
+    if (precision == DNSP_PRECISION_MIXED) b->tvar = 4;  // no workspace beside the FP32 fields
     b->nx.assign(nx, nx + n);
     b->nz.assign(nz, nz + n);
     b->ny.assign(ny, ny + n);
@@ -992,7 +987,6 @@ int dnsp_batch_create(int n, const int* nx, const int* nz, const int* ny, const 
     for (int i = 0; i < n; ++i) b->mr[(size_t)i] = part_rows_for(ny[i]);
     int rc = setup(b, bands);
     if (!rc) rc = setup_eig(b, inv_dx, inv_dz);
-    if (!rc) rc = setup_alone(b);
     if (!rc) rc = setup_groups(b);
     if (!rc) rc = upload_inst(b);
     if (rc) {
@@ -1020,6 +1014,8 @@ int dnsp_batch_bind(dnsp_batch* b, const double* const* rhs, double* const* P) {
     int rc = upload_inst(b);
     if (rc) return rc;
     b->bound = true;
+    // here, and not when the batch is created: the arrays come first
+    if (b->tvar == 6) alone_workspace(b);
     return DNSP_OK;
 }
 
@@ -1102,6 +1098,8 @@ int dnsp_batch_autotune(dnsp_batch* b, int reps, void* stream, double* times_ms)
         set_error("event creation failed");
         return DNSP_ERR_HIP;
     }
+    const bool had_w = b->d_W != nullptr;
+    alone_workspace(b);
     for (int form = 0; form < 2 && rc == DNSP_OK; ++form) {
         if (form == 1 && b->precision != DNSP_PRECISION_MIXED) break;
         int* var[3] = {form ? &b->mxvar : &b->xvar, form ? &b->mzvar : &b->zvar, form ? &b->mtvar : &b->tvar};
@@ -1138,6 +1136,10 @@ int dnsp_batch_autotune(dnsp_batch* b, int reps, void* stream, double* times_ms)
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
+    if (!had_w && b->tvar != 6) {  // not picked
+        (void)hipFree(b->d_W);     // (waits for the device)
+        b->d_W = nullptr;
+    }
     return rc;
 }
 

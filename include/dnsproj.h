@@ -260,23 +260,27 @@ int dnsp_poisson_mixed_info(const dnsp_poisson* h, int* fp32_on, double* f32_min
  *     precision as for dnsp_poisson_init (MIXED adds two FP32 fields per
  *     instance).
  *   dnsp_batch_bind: the device arrays of every instance (host arrays of n
- *     device pointers; rhs[i] != P[i], both 16-byte aligned); synchronous,
- *     done once.
+ *     device pointers; rhs[i] != P[i], both 16-byte aligned); synchronous.
+ *     Done once, or again when no run is in flight: later runs, and replays of
+ *     graphs captured before, use the new arrays.  Where tridiagonal variant 6
+ *     (below) is set, allocates its workspace if it can.
  *   dnsp_batch_run: FP64 solves P[i] = L_i^{-1} rhs[i] of all instances.
  *   dnsp_batch_run_mixed: mixed-precision solves, `refinements` 0 or 1.
  *   Both enqueue on `stream` only (no allocation, no synchronisation), so a
- *   caller may capture them in a graph.
+ *   caller may capture them in a graph.  Runs of one batch must not overlap:
+ *   they write the same arrays.
  *   dnsp_batch_autotune: times the whole batched solve per variant (x, z:
  *     0..3 as dnsp_poisson_set_variants; tridiagonal: 0 = 8-mode groups of
  *     32 chunks, 1 = the same with registers capped for 4 waves per SIMD, 2
  *     and 3 = 0 and 1 with two-pass chunks, 4 and 5 = 8-mode groups of 16
  *     chunks of twice the rows, one-pass and two-pass (32 chunks where the
- *     rows would exceed 32), 6 (FP64 only, the default) = 4, with the
- *     instances of 6 * 2^20 points and more solved one by one as
+ *     rows would exceed 32), 6 (FP64 form only; the default of an FP64 batch)
+ *     = 4, with the instances of 6 * 2^20 points and more solved one by one as
  *     dnsp_poisson_solve does, through one workspace of the largest's size
- *     that create allocates (as 4 if it cannot); x and z variants then apply
- *     to the smaller ones), keeps the fastest; overwrites the bound P
- *     arrays; times_ms as for dnsp_poisson_autotune.  Synchronises.
+ *     (as 4 without it); x and z variants then apply to the smaller ones),
+ *     keeps the fastest; overwrites the bound P arrays; times_ms as for
+ *     dnsp_poisson_autotune.  Allocates that workspace to time variant 6 and
+ *     frees it where another is kept.  Synchronises.
  *   dnsp_batch_set_variants / get_variants: FP64 x, z, tridiagonal, then the
  *     mixed form's (6 ints).
  */
