@@ -475,6 +475,22 @@ static int poisson_apply_strategy(dnsp_poisson* h) {
     return DNSP_OK;
 }
 
+// Values in (-1, 1) for the tuner's timed launches: on zeros, denormals or
+// infinities the kernels draw another power than in a solve.
+template <typename T>
+static __global__ __launch_bounds__(256) void k_tune_fill(T* __restrict__ a, long n) {
+    for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
+        unsigned long long z = (unsigned long long)i * 0x9E3779B97F4A7C15ull;
+        z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+        a[i] = (T)((double)(long long)(z ^ (z >> 27)) * 0x1p-63);
+    }
+}
+
+namespace dnsp {
+void tune_fill(double* a, size_t n, hipStream_t st) { k_tune_fill<<<2048, 256, 0, st>>>(a, (long)n); }
+void tune_fill(float* a, size_t n, hipStream_t st) { k_tune_fill<<<2048, 256, 0, st>>>(a, (long)n); }
+}  // namespace dnsp
+
 extern "C" {
 
 int dnsp_poisson_set_strategy(dnsp_poisson* h, int fft, int tridiag) {
@@ -529,21 +545,10 @@ int dnsp_poisson_get_variants(const dnsp_poisson* h, int* xvar, int* zvar, int* 
     return DNSP_OK;
 }
 
-// Values in (-1, 1) for the tuner's timed launches.  On zeros the kernels draw less
-// power and the order of two variants can change: at 768x384x384 the two-pass
-// tridiagonal was picked, 375-380 us inside a solve, over the one-pass one's 365.
-static __global__ __launch_bounds__(256) void k_tune_fill(double* __restrict__ a, long n) {
-    for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
-        unsigned long long z = (unsigned long long)i * 0x9E3779B97F4A7C15ull;
-        z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-        a[i] = (double)(long long)(z ^ (z >> 27)) * 0x1p-63;
-    }
-}
-
 // Times each FFT kernel variant per direction (`reps` forward transforms,
 // then `reps` inverse ones, keeping the fastest of each) and pairs of
-// tridiagonal solves per partitioned variant, on `work` (filled first;
-// NULL = a temporary device array); for a mixed-precision handle the same
+// tridiagonal solves per partitioned variant, on `work` (filled before every
+// kTuneRun calls; NULL = a temporary device array); for a mixed-precision handle the same
 // for its kernels.  times_ms (optional, DNSP_TUNE_SLOTS entries): mean ms of
 // a forward + inverse pair of the x, z (4 slots each) and of a pair of
 // tridiagonal (8 slots) variants, then the same for the mixed-precision
@@ -566,23 +571,12 @@ int dnsp_poisson_autotune(dnsp_poisson* h, double* work, int reps, void* stream,
     int* knob[5] = {&h->xvar, &h->xvar_b, &h->zvar, &h->zvar_b, &h->tvar};
     if (times_ms)
         for (int i = 0; i < DNSP_TUNE_SLOTS; ++i) times_ms[i] = -1.0;
-    auto timed = [&](int stage, int n, double* per) -> int {
-        (void)hipEventRecord(e0, st);
-        for (int r = 0; r < n; ++r) {
-            const int c = dnsp_poisson_stage(h, buf, buf, stage, stream);
-            if (c) return c;
-        }
-        (void)hipEventRecord(e1, st);
-        if (hipEventSynchronize(e1) != hipSuccess) {
-            set_error("autotune: event synchronize failed");
-            return DNSP_ERR_HIP;
-        }
-        float ms = 0.f;
-        (void)hipEventElapsedTime(&ms, e0, e1);
-        *per = (double)ms / n;
-        return DNSP_OK;
+    auto fill = [&]() { tune_fill(buf, N, st); };
+    auto timed = [&](int stage, double* per) -> int {
+        return tune_time(reps, kTuneRun, e0, e1, st, fill,
+                         [&]() { return dnsp_poisson_stage(h, buf, buf, stage, stream); }, per);
     };
-    auto fill = [&]() { k_tune_fill<<<2048, 256, 0, st>>>(buf, (long)N); };
+    fill();
     do {
         if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
             set_error("autotune: event creation failed");
@@ -599,12 +593,11 @@ int dnsp_poisson_autotune(dnsp_poisson* h, double* work, int reps, void* stream,
             for (int v = 0; v < nvar && rc == DNSP_OK; ++v) {
                 *knob[kf] = v;
                 *knob[kb] = v;
-                fill();  // repeated transforms scale the values
                 rc = dnsp_poisson_stage(h, buf, buf, sf, stream);  // warm-up
                 if (!rc) rc = dnsp_poisson_stage(h, buf, buf, sb, stream);
                 double tf = 0.0, tb = 0.0;
-                if (!rc) rc = timed(sf, reps, &tf);
-                if (!rc && dir < 2) rc = timed(sb, reps, &tb);
+                if (!rc) rc = timed(sf, &tf);
+                if (!rc && dir < 2) rc = timed(sb, &tb);
                 if (rc) break;
                 if (dir == 2) tf *= 2.0;  // a pair of tridiagonal solves, as the FFT pairs
                 if (times_ms) times_ms[kTuneSlot[dir] + v] = tf + tb;
@@ -621,24 +614,18 @@ int dnsp_poisson_autotune(dnsp_poisson* h, double* work, int reps, void* stream,
         if (rc || !h->blk_ok) break;
         // the blocked solve's own knobs, timed stage by stage through
         // dnsp_poisson_solve_stage on buf (rhs and solution) and the workspace; a
-        // stage leaves its input in place (the last one's scaled by each pass)
+        // stage leaves its input in place, but for the last one
         fill();
         const bool on = h->blk_on;
         h->blk_on = true;
         auto timed_b = [&](int stage, double* per) -> int {
-            int c = dnsp_poisson_solve_stage(h, buf, buf, stage, stream);  // warm-up
-            (void)hipEventRecord(e0, st);
-            for (int r = 0; r < reps && !c; ++r) c = dnsp_poisson_solve_stage(h, buf, buf, stage, stream);
+            const int c = dnsp_poisson_solve_stage(h, buf, buf, stage, stream);  // warm-up
             if (c) return c;
-            (void)hipEventRecord(e1, st);
-            if (hipEventSynchronize(e1) != hipSuccess) {
-                set_error("autotune: event synchronize failed");
-                return DNSP_ERR_HIP;
-            }
-            float ms = 0.f;
-            (void)hipEventElapsedTime(&ms, e0, e1);
-            *per = (double)ms / reps;
-            return DNSP_OK;
+            return tune_time(reps, stage == 4 ? kTuneRun : reps, e0, e1, st,
+                             [&]() {
+                                 if (stage == 4) fill();
+                             },
+                             [&]() { return dnsp_poisson_solve_stage(h, buf, buf, stage, stream); }, per);
         };
         int* bk[5] = {&h->bxvar, &h->bzvar, &h->btvar, &h->bzvar_b, &h->bxvar_b};  // by stage
         const int nv[5] = {kCtVariants, 2, kPartVariants, 2, kCtVariants};

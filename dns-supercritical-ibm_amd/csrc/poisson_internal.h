@@ -81,4 +81,40 @@ void mixed_release(dnsp_poisson* h);
 // Times the mixed-precision kernel variants and keeps the fastest.
 int mixed_autotune(dnsp_poisson* h, double* f, int reps, hipStream_t st, double* times_ms);
 
+// Fills an array for the tuner's timed launches.
+void tune_fill(double* a, size_t n, hipStream_t st);
+void tune_fill(float* a, size_t n, hipStream_t st);
+
+// Calls between two refills: an unnormalised transform in place multiplies the
+// values by the square root of its length, a solve or a scaled inverse divides
+// them, and hundreds in a row end in infinities or in zeros.
+constexpr int kTuneRun = 8;
+
+// Mean ms of `reps` calls of call() (an error code), in runs of about equal
+// length, at most `run`, each after an untimed refill().
+template <class F, class C>
+int tune_time(int reps, int run, hipEvent_t e0, hipEvent_t e1, hipStream_t st, const F& refill, const C& call,
+              double* per) {
+    const int runs = (reps + run - 1) / run;
+    double sum = 0.0;
+    for (int q = 0; q < runs; ++q) {
+        refill();
+        (void)hipEventRecord(e0, st);
+        for (int r = reps * q / runs; r < reps * (q + 1) / runs; ++r) {
+            const int c = call();
+            if (c) return c;
+        }
+        (void)hipEventRecord(e1, st);
+        if (hipGetLastError() != hipSuccess || hipEventSynchronize(e1) != hipSuccess) {
+            set_error("autotune: launch or synchronize failed");
+            return DNSP_ERR_HIP;
+        }
+        float ms = 0.f;
+        (void)hipEventElapsedTime(&ms, e0, e1);
+        sum += ms;
+    }
+    *per = sum / reps;
+    return DNSP_OK;
+}
+
 }  // namespace dnsp

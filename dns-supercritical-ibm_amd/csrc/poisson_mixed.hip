@@ -492,19 +492,17 @@ int mixed_autotune(dnsp_poisson* h, double* f, int reps, hipStream_t st, double*
         }
         mx_x_launch(kind, h->nx, v, a, st);
     };
+    const size_t N = (size_t)h->nx * h->nz * h->ny;
+    auto refill = [&]() {
+        tune_fill(f, N, st);
+        tune_fill(h->d_A, N, st);
+        tune_fill(h->d_B, N, st);
+    };
+    refill();
     auto time_of = [&](auto&& fn, double* per) -> int {
         fn();  // warm-up
-        (void)hipEventRecord(e0, st);
-        for (int r = 0; r < reps; ++r) fn();
-        (void)hipEventRecord(e1, st);
-        if (hipGetLastError() != hipSuccess || hipEventSynchronize(e1) != hipSuccess) {
-            set_error("mixed autotune: launch or synchronize failed");
-            return DNSP_ERR_HIP;
-        }
-        float ms = 0.f;
-        (void)hipEventElapsedTime(&ms, e0, e1);
-        *per = (double)ms / reps;
-        return DNSP_OK;
+        // half of kTuneRun: a call may run a kernel twice, in FP32's range
+        return tune_time(reps, kTuneRun / 2, e0, e1, st, refill, [&]() { return fn(), DNSP_OK; }, per);
     };
     int rc = DNSP_OK;
     // x: each kernel kind of the first two sweeps on its own
