@@ -577,6 +577,9 @@ int dnsp_poisson_autotune(dnsp_poisson* h, double* work, int reps, void* stream,
                          [&]() { return dnsp_poisson_stage(h, buf, buf, stage, stream); }, per);
     };
     fill();
+    // a work array that is not 16-byte aligned runs neither the compile-time x
+    // kernels nor the blocked solve: their knobs stay as they are
+    const bool al16 = (reinterpret_cast<uintptr_t>(buf) & 15) == 0;
     do {
         if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
             set_error("autotune: event creation failed");
@@ -584,7 +587,7 @@ int dnsp_poisson_autotune(dnsp_poisson* h, double* work, int reps, void* stream,
             break;
         }
         for (int dir = 0; dir < 3 && rc == DNSP_OK; ++dir) {
-            const bool has = dir == 0 ? h->ct_x : dir == 1 ? h->ct_z : h->part_rows > 0;
+            const bool has = dir == 0 ? h->ct_x && al16 : dir == 1 ? h->ct_z : h->part_rows > 0;
             if (!has) continue;
             const int nvar = dir == 2 ? kPartVariants : kCtVariants;
             const int sf = dir == 0 ? DNSP_STAGE_X_FWD : dir == 1 ? DNSP_STAGE_Z_FWD : DNSP_STAGE_TRIDIAG;
@@ -611,7 +614,7 @@ int dnsp_poisson_autotune(dnsp_poisson* h, double* work, int reps, void* stream,
                 }
             }
         }
-        if (rc || !h->blk_ok) break;
+        if (rc || !h->blk_ok || !al16) break;
         // the blocked solve's own knobs, timed stage by stage through
         // dnsp_poisson_solve_stage on buf (rhs and solution) and the workspace; a
         // stage leaves its input in place, but for the last one

@@ -35,3 +35,24 @@ def test_tuner_keeps_ordinary_values(cuda, nx, nz, ny, precision):
     r = r - r.mean()
     assert np.abs(g - g.mean() - r).max() <= 1e-12 * np.abs(r).max()
     s.close()
+
+
+def test_tuner_on_an_array_aligned_to_eight_bytes(cuda):
+    """A work array that is not 16-byte aligned runs other x kernels and no blocked
+    solve: those knobs are not timed and stay as they were set."""
+    import torch
+    nx, nz, ny = 128, 64, 40
+    print("[gpu-case] tuner, 8-byte aligned work", flush=True)
+    yu = W.tanh_faces(ny, 1.4)
+    bands = D.mk_P_abc(yu, False) + D.mk_P_abc(yu, True)
+    s = D.PoissonSolver(nx, nz, ny, nx / W.LX, nz / W.LZ, bands)
+    work = torch.zeros(nx * nz * ny + 1, dtype=torch.float64, device="cuda:0")[1:].view(ny, nz, nx)
+    assert work.data_ptr() % 16 == 8
+    for xv, zv, tv in ((1, 0, 1), (3, 1, 5)):
+        s.set_variants(xv, zv, tv)
+        before = s.solve_variants
+        t = s.autotune(work=work, reps=3)
+        assert s.solve_variants == before
+        assert t["x_ms"] == [-1.0] * 4 and t["picked"][0] == xv
+        assert min(t["z_ms"]) > 0 and min(t["tri_ms"]) > 0
+    s.close()
