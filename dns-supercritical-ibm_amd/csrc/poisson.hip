@@ -458,8 +458,8 @@ static int poisson_apply_strategy(dnsp_poisson* h) {
         DNSP_HIP_TRY(hipMalloc(&h->d_cp, sizeof(double) * N));
     }
     const bool rg = h->fft_strategy == DNSP_FFT_AUTO;
-    h->rx = rg && !h->ct_x ? rg_ops(h->nx) : nullptr;
-    h->rz = rg && !h->ct_z ? rg_ops(h->nz) : nullptr;
+    h->rx = rg ? rg_ops(h->nx) : nullptr;
+    h->rz = rg ? rg_ops(h->nz) : nullptr;
     // the blocked solve: compile-time x and z transforms (all their lengths are
     // multiples of 16), the partitioned tridiagonal; its workspace is one field.
     // Not with register-direct transforms: a handle of such lengths writes the
@@ -724,12 +724,12 @@ int dnsp_poisson_stage(dnsp_poisson* h, const double* src, double* P, int stage,
     switch (stage) {
         case DNSP_STAGE_X_FWD:
             if (h->ct_x && x16) ct_x_launch(h->nx, h->xvar, false, src, P, nlines, h->d_twx, 1.0, st);
-            else if (h->rx) h->rx->xfwd(src, P, nlines, h->nz, (long)h->nx * h->nz, h->nx, 16, h->d_twx, st);
+            else if (h->rx) h->rx->xfwd(src, P, nlines, h->d_twx, st);
             else k_xfwd<<<gx, kFftThreads, ldsx, st>>>(src, P, h->nx, nlines, h->Gx, h->px);
             break;
         case DNSP_STAGE_Z_FWD:
             if (h->ct_z) ct_z_launch(h->nz, h->zvar, false, P, h->nx, h->ny, h->d_twz, st);
-            else if (h->rz) h->rz->zfwd(P, P, h->nx, h->ny, (long)h->nx * h->nz, 16, h->nx, 0, h->d_twz, st);
+            else if (h->rz) h->rz->zfwd(P, h->nx, h->ny, h->d_twz, st);
             else k_zfwd<<<gz, kFftThreads, ldsz, st>>>(P, h->nx, h->nz, h->ncol, h->TAz, h->pz);
             break;
         case DNSP_STAGE_TRIDIAG: {
@@ -746,7 +746,7 @@ int dnsp_poisson_stage(dnsp_poisson* h, const double* src, double* P, int stage,
         }
         case DNSP_STAGE_Z_BWD:
             if (h->ct_z) ct_z_launch(h->nz, h->zvar_b, true, P, h->nx, h->ny, h->d_twz, st);
-            else if (h->rz) h->rz->zbwd(P, P, h->nx, h->ny, (long)h->nx * h->nz, 16, h->nx, h->d_twz, st);
+            else if (h->rz) h->rz->zbwd(P, h->nx, h->ny, h->d_twz, st);
             else k_zbwd<<<gz, kFftThreads, ldsz, st>>>(P, h->nx, h->nz, h->ncol, h->TAz, h->pz);
             break;
         case DNSP_STAGE_X_BWD:

@@ -8,7 +8,12 @@
 
 namespace dnsp {
 
-bool ct_fft_supported(int n);
+// The lengths with compile-time-sized kernels.
+constexpr bool ct_fft_supported(int n) {
+    for (int m : {32, 64, 96, 128, 192, 256, 384, 512, 768})
+        if (n == m) return true;
+    return false;
+}
 // at (inverse only; device, NULL: src and dst): the place of the address of the
 // array to transform in place, read when the kernel runs (array_at).
 void ct_x_launch(int n, int variant, bool inv, const double* src, double* dst, long nlines, const double2* tw,
@@ -23,24 +28,20 @@ void xb_x_launch(int n, int variant, const double* src, double* dst, long nlines
                  hipStream_t st, const double* const* at = nullptr);
 void mm_z_launch(int n, int variant, bool inv, const double* src, double* dst, int nx, int ny, const double2* tw,
                  hipStream_t st, double* const* at = nullptr);
-// The FP64 transforms of every length 16..768 with prime factors up to 13
-// (poisson_reg.h; strides and layouts there).  z: mm = 1 writes the
-// mode-major blocks, 0 back in place.
+// The in-place FP64 transforms of the other lengths 16..768 with prime factors up
+// to 13 (poisson_reg.h).
 constexpr int kRgMin = 16, kRgMax = 768;
 constexpr bool rg_supported(int n) {
-    if (n < kRgMin || n > kRgMax) return false;
+    if (n < kRgMin || n > kRgMax || ct_fft_supported(n)) return false;
     for (int p : {2, 3, 5, 7, 11, 13})
         while (n % p == 0) n /= p;
     return n == 1;
 }
 struct RgOps {
-    void (*xfwd)(const double* P, double* S, long nlines, int nz, long sk, int sj, int sb, const double2* tw,
-                 hipStream_t st);
+    void (*xfwd)(const double* P, double* S, long nlines, const double2* tw, hipStream_t st);
     void (*xbwd)(const double* S, double* P, long nlines, double scale, const double2* tw, hipStream_t st);
-    void (*zfwd)(const double* src, double* dst, int nx, int ny, long sk, int sc, int sj, int mm, const double2* tw,
-                 hipStream_t st);
-    void (*zbwd)(const double* src, double* dst, int nx, int ny, long sk, int sc, int sj, const double2* tw,
-                 hipStream_t st);
+    void (*zfwd)(double* S, int nx, int ny, const double2* tw, hipStream_t st);
+    void (*zbwd)(double* S, int nx, int ny, const double2* tw, hipStream_t st);
 };
 const RgOps* rg_ops(int n);  // NULL where not supported
 // The x variants the blocked solve starts with (us).  Forward: 1536 complex

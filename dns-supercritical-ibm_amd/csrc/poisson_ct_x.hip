@@ -6,16 +6,6 @@ namespace dnsp {
 
 #define DNSP_CT_SIZES(X) X(32) X(64) X(96) X(128) X(192) X(256) X(384) X(512) X(768)
 
-bool ct_fft_supported(int n) {
-    switch (n) {
-#define DNSP_CASE(N) case N:
-        DNSP_CT_SIZES(DNSP_CASE)
-#undef DNSP_CASE
-        return true;
-        default: return false;
-    }
-}
-
 template <int N, int V>
 static void ct_x(bool inv, const double* src, double* dst, long nlines, const double2* tw, double scale,
                  hipStream_t st, double* const* at) {

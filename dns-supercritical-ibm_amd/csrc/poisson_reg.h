@@ -1,23 +1,18 @@
-// Transform kernels of the FP64 Poisson solve on the register-direct FFT
-// (fft_reg.h), for every length 16..768 with prime factors up to 13.  Layout
-// strides are arguments, so one kernel serves the in-place stages and the
-// blocked solve.
-//
-// Layouts of a field (element of halfcomplex x row a, z index j, plane k):
-//   lines       k nz nx + j nx + a                    (the caller's array)
-//   x-blocked   ((k nx/16 + a/16) nz + j) 16 + a%16   (the workspace; nx % 16 == 0)
-//   mode-major  ((a/16 nz + j) ny + k) 16 + a%16      (the caller's array; nx % 16 == 0)
+// In-place transform kernels of the FP64 Poisson solve on the register-direct FFT
+// (fft_reg.h), for the lengths 16..768 with prime factors up to 13 that have no
+// kernels in poisson_ct.h.  Element of x row a, z index j, plane k of a field
+// (the caller's array): k nz nx + j nx + a.
 //
 // Bound: HBM (one read and one write of the field).  Measured on one MI355X,
-// x forward / z forward / z inverse / x inverse in us, against the
-// runtime-sized kernels of poisson.hip, which these lengths ran before (they
-// divide per element, load 8 bytes at a time under branches and gather their
-// twiddles): 560 x 280 x 280 (0.70 GB a kernel) 155 / 137 / 129 / 146 against
-// 560 / 618 / 432 / 409 (4.5-5.4 TB/s); 624 x 312 x 770 x forward 0.51 ms
-// against 1.99.  At the lengths of poisson_ct.h (768 x 384 x 384: 376 / 353 /
-// 315 / 323, 256 x 128 x 192: 21 / 17.5 / 16.4 / 19.5) they are within 5% of
-// the best variant there on either side, so those lengths keep their tuned
-// variants.
+// x forward / z forward / z inverse / x inverse in us (mean of 12 solves under
+// the profiler), against the runtime-sized kernels of poisson.hip, which these
+// lengths ran before (they divide per element, load 8 bytes at a time under
+// branches and gather their twiddles): 560 x 280 x 280 (0.70 GB a kernel) 170 /
+// 152 / 138 / 164 against 560 / 618 / 432 / 409 (4.1-5.1 TB/s); 624 x 312 x 770
+// (2.4 GB) 502 / 426 / 415 / 539, x forward against 1990.  At the lengths of
+// poisson_ct.h they were within 5% of the best variant there on either side
+// (in the blocked layouts, 768 x 384 x 384: 376 / 353 / 315 / 323), so those
+// lengths keep their tuned variants and have no kernels here.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -55,19 +50,17 @@ constexpr int kRgCols = 8;
 // (fastest over lanes) and two neighbouring elements fall on different banks.
 constexpr int rg_col_pitch(int n) { return ct_pitch(n) + (18 - ct_pitch(n) % 16) % 16; }
 
-// x forward: lines -> element a of line (j, k) at k sk + j sj + (a/16) sb + a%16.
+// x forward, lines -> lines (in place allowed).
 template <int N, int G, int NT>
-__global__ __launch_bounds__(NT) void kr_xfwd(const double* P, double* S, long nlines,
-                                              int nz, long sk, int sj, int sb, const double2* __restrict__ tw) {
+__global__ __launch_bounds__(NT) void kr_xfwd(const double* P, double* S, long nlines, const double2* __restrict__ tw) {
     constexpr int LP = ct_pitch(N);
     __shared__ double2 buf[G * LP];
     __shared__ double2 stw[N];
     ct_stage_twiddles<N, NT>(stw, tw);
     const long l0 = (long)xcd_tile(blockIdx.x, gridDim.x) * 2 * G;
     const int left = nlines - l0 < 2 * G ? (int)(nlines - l0) : 2 * G;  // valid lines of this tile
-    const int kb = (int)(l0 / nz), jb = (int)(l0 - (long)kb * nz);
-    const unsigned long long mz = line_div_magic(nz);
     const double* src = P + l0 * N;
+    double* dst = S + l0 * N;
     auto ld = [&](int g, int j, int m, auto& v) {
         constexpr int R = sizeof(v) / sizeof(v[0]);
         const int la = 2 * g < left ? 2 * g : 0;
@@ -81,23 +74,15 @@ __global__ __launch_bounds__(NT) void kr_xfwd(const double* P, double* S, long n
 #pragma unroll
         for (int r = 0; r < R; ++r) v[r].y = vb ? v[r].y : 0.0;
     };
-    double* dst = S + kb * sk;
-    const unsigned skb = (unsigned)sk * 8u;
     auto st = [&](int g, int lo, int hi, bool both, double2 L, double2 H) {
         if (2 * g >= left) return;
-        int k, j;
-        tile_line_kj(0, jb, 2 * g, nz, mz, k, j);
-        const unsigned oa = (unsigned)k * skb + (unsigned)(j * sj) * 8u;
-        const bool wrap = j + 1 == nz;
-        const unsigned ob = wrap ? (unsigned)(k + 1) * skb : oa + (unsigned)sj * 8u;
+        const unsigned oa = (unsigned)(2 * g * N) * 8u, ob = oa + N * 8u;
         const bool vb = 2 * g + 1 < left;
-        const unsigned el = ((unsigned)(lo >> 4) * (unsigned)sb + (unsigned)(lo & 15)) * 8u;
-        rg_st(dst, oa + el, L.x);
-        if (vb) rg_st(dst, ob + el, L.y);
+        rg_st(dst, oa + (unsigned)lo * 8u, L.x);
+        if (vb) rg_st(dst, ob + (unsigned)lo * 8u, L.y);
         if (both) {
-            const unsigned eh = ((unsigned)(hi >> 4) * (unsigned)sb + (unsigned)(hi & 15)) * 8u;
-            rg_st(dst, oa + eh, H.x);
-            if (vb) rg_st(dst, ob + eh, H.y);
+            rg_st(dst, oa + (unsigned)hi * 8u, H.x);
+            if (vb) rg_st(dst, ob + (unsigned)hi * 8u, H.y);
         }
     };
     rg_forward<N, G, NT, LP, false>(buf, stw, ld, st);
@@ -138,11 +123,10 @@ __global__ __launch_bounds__(NT) void kr_xbwd(const double* S, double* P, long n
     rg_inverse<N, G, NT, LP, false>(buf, stw, ld, st);
 }
 
-// z kernels: one workgroup per (plane k, block c of 16 x rows); complex column g
-// pairs rows 16c + 2g and 16c + 2g + 1 (the last row of an odd nx is paired
-// with zero).  Input element (j, g) at k sk + c sc + j sj + 2g.  A pair is one
-// 16-byte access where all pairs are 16-byte aligned (even strides, aligned
-// array; uniform over the grid), else two 8-byte ones.
+// z kernels, in place: one workgroup per (plane k, block c of 16 x rows); complex
+// column g pairs rows 16c + 2g and 16c + 2g + 1 (the last row of an odd nx is
+// paired with zero).  A pair is one 16-byte access where all pairs are 16-byte
+// aligned (even nx, aligned array; uniform over the grid), else two 8-byte ones.
 __device__ __forceinline__ double2 rg_ldp(const double* base, unsigned off, bool al, bool two) {
     if (al) return rg_ld2(base, off);
     const double a = rg_ld(base, off), b = rg_ld(base, two ? off + 8u : off);
@@ -156,13 +140,10 @@ __device__ __forceinline__ void rg_stp(double* base, unsigned off, bool al, bool
         if (two) rg_st(base, off + 8u, v.y);
     }
 }
-__device__ __forceinline__ bool rg_pairs_aligned(const void* p, long sk, int sj) {
-    return ((size_t)p & 15) == 0 && ((sk | sj) & 1) == 0;
-}
+__device__ __forceinline__ bool rg_pairs_aligned(const void* p, int nx) { return ((size_t)p & 15) == 0 && nx % 2 == 0; }
 
 template <int N, int NT>
-__global__ __launch_bounds__(NT) void kr_zfwd(const double* src, double* dst, int nx, int ny, long sk, int sc, int sj,
-                                              int mm, const double2* __restrict__ tw) {
+__global__ __launch_bounds__(NT) void kr_zfwd(double* S, int nx, const double2* __restrict__ tw) {
     constexpr int G = kRgCols, LP = rg_col_pitch(N);
     __shared__ double2 buf[G * LP];
     __shared__ double2 stw[N];
@@ -171,31 +152,26 @@ __global__ __launch_bounds__(NT) void kr_zfwd(const double* src, double* dst, in
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
     const int k = tile / nab, c = tile - k * nab;
     const int w = nx - 16 * c < 16 ? nx - 16 * c : 16;  // rows of the block
-    const bool al = rg_pairs_aligned(src, sk, sj) && rg_pairs_aligned(dst, sk, sj);
-    const double* s = src + k * sk + (long)c * sc;
-    const unsigned sjb = (unsigned)sj * 8u;
+    const bool al = rg_pairs_aligned(S, nx);
+    double* s = S + (long)k * nx * N + 16 * c;
+    const unsigned nxb = (unsigned)nx * 8u;
     auto ld = [&](int g, int j, int m, auto& v) {
         constexpr int R = sizeof(v) / sizeof(v[0]);
         const int gg = 2 * g < w ? g : 0;
-        const unsigned o = (unsigned)j * sjb + (unsigned)gg * 16u, ms = (unsigned)m * sjb;
+        const unsigned o = (unsigned)j * nxb + (unsigned)gg * 16u, ms = (unsigned)m * nxb;
 #pragma unroll
         for (int r = 0; r < R; ++r) v[r] = rg_ldp(s, o + (unsigned)r * ms, al, 2 * gg + 1 < w);
     };
-    // mode-major (mm), or back in place
-    double* d = mm ? dst + (long)c * N * ny * 16 + (long)k * 16 : dst + k * sk + (long)c * sc;
-    const unsigned sbb = mm ? (unsigned)ny * 128u : sjb;
     auto st = [&](int g, int lo, int hi, bool both, double2 L, double2 H) {
         if (2 * g >= w) return;
-        rg_stp(d, (unsigned)lo * sbb + (unsigned)g * 16u, al, 2 * g + 1 < w, L);
-        if (both) rg_stp(d, (unsigned)hi * sbb + (unsigned)g * 16u, al, 2 * g + 1 < w, H);
+        rg_stp(s, (unsigned)lo * nxb + (unsigned)g * 16u, al, 2 * g + 1 < w, L);
+        if (both) rg_stp(s, (unsigned)hi * nxb + (unsigned)g * 16u, al, 2 * g + 1 < w, H);
     };
     rg_forward<N, G, NT, LP, true>(buf, stw, ld, st);
 }
 
-// z inverse -> lines.
 template <int N, int NT>
-__global__ __launch_bounds__(NT) void kr_zbwd(const double* src, double* dst, int nx, long sk, int sc, int sj,
-                                              const double2* __restrict__ tw) {
+__global__ __launch_bounds__(NT) void kr_zbwd(double* S, int nx, const double2* __restrict__ tw) {
     constexpr int G = kRgCols, LP = rg_col_pitch(N);
     __shared__ double2 buf[G * LP];
     __shared__ double2 stw[N];
@@ -204,22 +180,20 @@ __global__ __launch_bounds__(NT) void kr_zbwd(const double* src, double* dst, in
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
     const int k = tile / nab, c = tile - k * nab;
     const int w = nx - 16 * c < 16 ? nx - 16 * c : 16;
-    const bool al = rg_pairs_aligned(src, sk, sj) && rg_pairs_aligned(dst, nx, nx);
-    const double* s = src + k * sk + (long)c * sc;
-    const unsigned sjb = (unsigned)sj * 8u;
+    const bool al = rg_pairs_aligned(S, nx);
+    double* s = S + (long)k * nx * N + 16 * c;
+    const unsigned nxb = (unsigned)nx * 8u;
     auto ld = [&](int g, int lo, int hi, double2& A, double2& B) {
         const int gg = 2 * g < w ? g : 0;
-        A = rg_ldp(s, (unsigned)lo * sjb + (unsigned)gg * 16u, al, 2 * gg + 1 < w);
-        B = rg_ldp(s, (unsigned)hi * sjb + (unsigned)gg * 16u, al, 2 * gg + 1 < w);
+        A = rg_ldp(s, (unsigned)lo * nxb + (unsigned)gg * 16u, al, 2 * gg + 1 < w);
+        B = rg_ldp(s, (unsigned)hi * nxb + (unsigned)gg * 16u, al, 2 * gg + 1 < w);
     };
-    double* d = dst + (long)k * nx * N + 16 * c;
-    const unsigned nxb = (unsigned)nx * 8u;
     auto st = [&](int g, int j, int m, auto& v) {
         constexpr int R = sizeof(v) / sizeof(v[0]);
         if (2 * g >= w) return;
         const unsigned o = (unsigned)j * nxb + (unsigned)g * 16u, ms = (unsigned)m * nxb;
 #pragma unroll
-        for (int r = 0; r < R; ++r) rg_stp(d, o + (unsigned)r * ms, al, 2 * g + 1 < w, v[r]);
+        for (int r = 0; r < R; ++r) rg_stp(s, o + (unsigned)r * ms, al, 2 * g + 1 < w, v[r]);
     };
     rg_inverse<N, G, NT, LP, true>(buf, stw, ld, st);
 }

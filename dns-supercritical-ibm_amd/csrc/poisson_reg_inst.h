@@ -13,20 +13,18 @@ namespace {
 template <int N>
 struct RgLaunch {
     static constexpr int G = rg_x_lines(N), NTX = rg_threads(G * N), NTZ = rg_threads(kRgCols * N);
-    static void xfwd(const double* P, double* S, long nlines, int nz, long sk, int sj, int sb, const double2* tw,
-                     hipStream_t st) {
-        kr_xfwd<N, G, NTX><<<(int)((nlines + 2 * G - 1) / (2 * G)), NTX, 0, st>>>(P, S, nlines, nz, sk, sj, sb, tw);
+    static int lines_blocks(long nlines) { return (int)((nlines + 2 * G - 1) / (2 * G)); }
+    static void xfwd(const double* P, double* S, long nlines, const double2* tw, hipStream_t st) {
+        kr_xfwd<N, G, NTX><<<lines_blocks(nlines), NTX, 0, st>>>(P, S, nlines, tw);
     }
     static void xbwd(const double* S, double* P, long nlines, double scale, const double2* tw, hipStream_t st) {
-        kr_xbwd<N, G, NTX><<<(int)((nlines + 2 * G - 1) / (2 * G)), NTX, 0, st>>>(S, P, nlines, scale, tw);
+        kr_xbwd<N, G, NTX><<<lines_blocks(nlines), NTX, 0, st>>>(S, P, nlines, scale, tw);
     }
-    static void zfwd(const double* src, double* dst, int nx, int ny, long sk, int sc, int sj, int mm,
-                     const double2* tw, hipStream_t st) {
-        kr_zfwd<N, NTZ><<<(nx + 15) / 16 * ny, NTZ, 0, st>>>(src, dst, nx, ny, sk, sc, sj, mm, tw);
+    static void zfwd(double* S, int nx, int ny, const double2* tw, hipStream_t st) {
+        kr_zfwd<N, NTZ><<<(nx + 15) / 16 * ny, NTZ, 0, st>>>(S, nx, tw);
     }
-    static void zbwd(const double* src, double* dst, int nx, int ny, long sk, int sc, int sj, const double2* tw,
-                     hipStream_t st) {
-        kr_zbwd<N, NTZ><<<(nx + 15) / 16 * ny, NTZ, 0, st>>>(src, dst, nx, sk, sc, sj, tw);
+    static void zbwd(double* S, int nx, int ny, const double2* tw, hipStream_t st) {
+        kr_zbwd<N, NTZ><<<(nx + 15) / 16 * ny, NTZ, 0, st>>>(S, nx, tw);
     }
 };
 
