@@ -32,8 +32,7 @@ struct dnsp_step {
     double* f[DNSP_STEP_NFIELDS] = {};  // halo fields, then P (interior)
     double* d_geom = nullptr;           // inv_dy_p (ny), inv_dy_p_pad (ny+1), hi (ny), lo (ny)
     double* d_rho_min = nullptr;        // 1
-    double* d_walls = nullptr;          // 6: U_bot, V_bot, W_bot, U_top, V_top, W_top
-    double walls[6] = {0, 0, 0, 0, 0, 0};
+    double walls[6] = {0, 0, 0, 0, 0, 0};  // U_bot, V_bot, W_bot, U_top, V_top, W_top
     dnsp_ibm* ibm[3] = {nullptr, nullptr, nullptr};  // U, V, W (borrowed)
     int* d_bot[3] = {};                 // rough-wall column slabs of U, V, W (nx*nz each), or NULL
     int* d_top[3] = {};
@@ -53,7 +52,6 @@ void release(dnsp_step* s) {
     for (double*& p : s->f) (void)hipFree(p);
     (void)hipFree(s->d_geom);
     (void)hipFree(s->d_rho_min);
-    (void)hipFree(s->d_walls);
     for (int c = 0; c < 3; ++c) {
         (void)hipFree(s->d_bot[c]);
         (void)hipFree(s->d_top[c]);
@@ -172,15 +170,13 @@ int dnsp_step_create(int nx, int nz, int ny, const double* yu, double inv_dx, do
         ok = ok && hipMalloc(&s->d_geom, sizeof(double) * g.size()) == hipSuccess &&
              hipMemcpy(s->d_geom, g.data(), sizeof(double) * g.size(), hipMemcpyHostToDevice) == hipSuccess &&
              hipMalloc(&s->d_rho_min, sizeof(double)) == hipSuccess &&
-             hipMemset(s->d_rho_min, 0, sizeof(double)) == hipSuccess &&
-             hipMalloc(&s->d_walls, sizeof(double) * 6) == hipSuccess &&
-             hipMemset(s->d_walls, 0, sizeof(double) * 6) == hipSuccess;
+             hipMemset(s->d_rho_min, 0, sizeof(double)) == hipSuccess;
         if (!ok) {
             set_error("device allocation of the step fields failed");
             rc = DNSP_ERR_NOMEM;
             break;
         }
-        s->bytes += sizeof(double) * (g.size() + 7);
+        s->bytes += sizeof(double) * (g.size() + 1);
     } while (0);
     if (rc) {
         release(s);
@@ -238,7 +234,6 @@ int dnsp_step_set_walls(dnsp_step* s, const double* wall_bc) {
     clear_error();
     DNSP_ARG_CHECK(s && wall_bc, "NULL argument");
     std::memcpy(s->walls, wall_bc, sizeof(s->walls));
-    DNSP_HIP_TRY(hipMemcpy(s->d_walls, wall_bc, sizeof(double) * 6, hipMemcpyHostToDevice));
     return DNSP_OK;
 }
 
