@@ -857,10 +857,10 @@ int upload_inst(dnsp_batch* b) {
 void run_alone(const BInst& I, BInst* d, double* W, hipStream_t st) {
     xb_x_launch(I.nx, blk_xfwd_variant(points(I)), nullptr, W, I.nlines, I.nz, I.twx, st, &d->f);
     mm_z_launch(I.nz, kBlkZVariant, false, W, nullptr, I.nx, I.ny, I.twz, st, &d->P);
-    static_assert(kPartDefault == 2, "one-pass rule-shaped tridiagonal");
+    static_assert(kPartDefault == 2, "rule-shaped tridiagonal");
     PartArgs<double> t{nullptr, I.ax, I.az, I.bands, I.nx, I.nz, I.ny, I.pcr_min, nullptr, nullptr, 0.0, nullptr, 0, W,
                        &d->P};
-    part_launch_rule<double, double, false, true>(t, st);
+    part_launch_rule<double, double, true>(t, st);
     mm_z_launch(I.nz, kBlkZVariant, true, W, nullptr, I.nx, I.ny, I.twz, st, &d->P);
     ct_x_launch(I.nx, blk_xbwd_variant(I.nx), true, nullptr, nullptr, I.nlines, I.twx, I.inv_nxnz, st, &d->P);
 }

@@ -61,7 +61,7 @@ void ct_z_launch(int n, int variant, bool inv, float* S, int nx, int ny, const f
 // per mode of up to 32 rows, M modes per workgroup), FP64 spectra: 0 = P 32, M
 // 16, registers capped for 4 resident waves per SIMD; 1 = P 32, M 8; 2 = the
 // shape part_shape gives ny, with exactly ceil(ny / P) rows a chunk; 3 = P 16, M
-// 16 (ny <= 512, else P 64, M 8); 4..7 = the same with two-pass chunks.
+// 16 (ny <= 512, else P 64, M 8); 4, 5, 7 = 0, 1, 3 with two-pass chunks; 6 = 2.
 constexpr int kPartChunks = 32;
 constexpr int kPartVariants = 8;
 // tuner table: first slot of the x, z and tridiagonal variants of one form
@@ -70,18 +70,23 @@ constexpr int kTuneFormSlots = 16;
 int part_rows_for(int ny);  // rows per chunk at kPartChunks chunks (0: ny too large)
 // Chunks per mode by ny.  Fewer chunks shorten the reduced system (its
 // log2(P) barrier steps, and the serial sweep of the low modes) and move less
-// through LDS; more rows a chunk take more registers (about 6 VGPRs a row, 8 in
-// the two-pass form), hence fewer resident waves.  Measured per launch
-// (576 x 288 modes; us, fraction of 5.4 TB/s), against the 32 x 16 shape with
-// its rows rounded up to {2,3,4,6,8,12,16,24,32} that ran before:
-//   ny  33  P 4: 17.7 (0.92)  P 8: 18.9  P 16: 31.0  before 65
-//   ny  65  P 8: 29.2 (1.09)  P 4: 29.7  P 16: 35.5  before 66
-//   ny 129  P 16: 68.8 (0.92) P 8: 69.5              before 103
-//   ny 280  P 16: 146 (0.94)  P 32: 149              before 230 (384 rows)
-//   ny 384  P 16: 201 (0.94)  P 32: 203              before 247
-//   ny 770  P 32, M 8: 455 (0.83)  M 16: 555  P 16: 959  before 1403
+// through LDS; more rows a chunk take more registers (about 6 VGPRs a row), hence
+// fewer resident waves.  us per launch, one pass, 576 x 288 modes in mode-major
+// blocks, by P:
+//   ny  33  P 4  17.7  P 8  18.9  P 16 31.0
+//   ny  65  P 8  29.2  P 4  29.7  P 16 35.5
+//   ny 129  P 16 68.8  P 8  69.5  P 12 70.4
+//   ny 280  P 16 146   P 32 150   P 24 183
+//   ny 384  P 16 206   P 32 206   P 24 297
+//   ny 770  P 32, M 8 477   M 16 555   P 24, M 8 461   P 16 959
+// Inside the library, the shape against (32, 16) with its rows rounded up to {2,
+// 3, 4, 6, 8, 12, 16, 24, 32}, in place at 576 x 288 modes and in the blocked layouts
+// at 768 x 192: ny 33 18 / 67 and 16 / 58, 65 31 / 69 and 28 / 62, 129 57 / 95 and 64 /
+// 100, 280 159 / 218 and 138 / 192, 384 236 / 254 and 196 / 227, 512 301 / 314 and
+// 242 / 272, 770 584 / 1620 (3.5 TB/s) and 504 / 1403.
 // Above 512 rows two workgroups of 16 modes no longer fit a CU's registers, so
-// a workgroup holds 8.  FP32 spectra take twice the modes: 32 make 128-byte rows.
+// a workgroup holds 8, whose rows are half a cache line.  FP32 spectra take twice
+// the modes: 32 make 128-byte rows.
 struct PartShape {
     int P, M, MR;
 };
@@ -90,11 +95,13 @@ constexpr PartShape part_shape(int ny, bool fp32 = false) {
     const int mr = (ny + P - 1) / P;
     return {P, (P == 32 ? 8 : 16) * (fp32 ? 2 : 1), mr < 2 ? 2 : mr};
 }
-// The variant a handle starts with, FP32 or FP64 spectra: part_shape's,
-// one-pass.  Two passes save registers but solve a chunk's interior again;
-// measured (us, one- against two-pass; mode-major and in place): 384x192x336
-// 84/86 and 65/72, 384x192x512 131/136 and 152/153, 576x288x400 220/242 and
-// 244/249, 624x312x770 657/722 and 679/752, 96x48x1000 33/35 and 32/36.
+// The variant a handle starts with, FP32 or FP64 spectra: part_shape's, one-pass.
+// Two passes save registers but solve a chunk's interior again, and were 2-11%
+// slower (us, one / two passes; in place at 576 x 288 modes: ny 65 31 / 32, 280 159 /
+// 167, 384 236 / 244, 512 301 / 308, 770 584 / 645; blocked at 768 x 192: 65 27.5 / 28.7,
+// 129 64 / 63, 280 138 / 143, 384 196 / 213, 512 242 / 254, 770 504 / 561; a whole
+// mixed solve of 512x256x256 692 / 702, 384x192x600 1139 / 1215), so the shape has no
+// two-pass form and variant 6 runs the same kernels.
 constexpr int kPartDefault = 2;
 // The group lists of an FP32-spectrum variant (the mixed form launches the
 // well-conditioned groups in FP32 arithmetic and the rest in FP64): 0 = groups
@@ -121,7 +128,7 @@ struct PartArgs {
     T* So;
     T* const* at = nullptr;  // MM: the place of S's address, as ct_x_launch
 };
-template <typename T, typename Ar, bool TP, bool MM>
+template <typename T, typename Ar, bool MM>
 void part_launch_rule(const PartArgs<T>& a, hipStream_t st);
 template <typename T, typename Ar = double, bool MM = false>
 void part_launch(int variant, T* S, const double* ax, const double* az, const double* bands, int nx, int nz,

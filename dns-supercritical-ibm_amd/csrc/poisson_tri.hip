@@ -65,8 +65,7 @@ void part_launch(int variant, T* S, const double* ax, const double* az, const do
                                              nlist, So)
     if (variant == 2 || variant == 6) {
         const PartArgs<T> a{S, ax, az, bands, nx, nz, ny, pcr_min, msum, pbar, inv_nxnz, glist, nlist, So};
-        if (variant == 2) part_launch_rule<T, Ar, false, MM>(a, st);
-        else part_launch_rule<T, Ar, true, MM>(a, st);
+        part_launch_rule<T, Ar, MM>(a, st);
         return;
     }
     if constexpr (sizeof(T) == 4) {

@@ -1,6 +1,5 @@
 // One-pass rule-shaped tridiagonal kernels, in place.
 #define DNSP_RULE_T double
 #define DNSP_RULE_AR double
-#define DNSP_RULE_TP false
 #define DNSP_RULE_MM false
 #include "poisson_tri_rule.h"

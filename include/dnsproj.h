@@ -182,10 +182,10 @@ int dnsp_poisson_get_strategy(const dnsp_poisson* h, int* fft_ct_x, int* fft_ct_
  * (32, 8) (1), a shape by ny with exactly ceil(ny / chunks) rows (4, 8 or 16
  * chunks of 16 modes up to 48, 128 and 512 rows, 32 chunks of 8 modes above)
  * (2), (16, 16) for ny <= 512, else (64, 8) (3); rows per chunk follow from ny.
- * 4..7: the same shapes with two-pass chunks (the chunk interior is solved
- * again once its end values are known, instead of being kept in registers
- * across the reduced solve).  A handle starts with 2.  The mixed-precision
- * form has its own set; on its FP32 spectra shapes 2 and 6 have twice the modes
+ * 4, 5, 7: the shapes of 0, 1, 3 with two-pass chunks (the chunk interior is
+ * solved again once its end values are known, instead of being kept in
+ * registers across the reduced solve); 6: as 2.  A handle starts with 2.  The mixed-precision
+ * form has its own set; on its FP32 spectra shape 2 has twice the modes
  * (32, and 16 above 512 rows), 3 and 7 are (16, 32): 32 modes make 128-byte
  * rows.  No counterpart in the reference. */
 int dnsp_poisson_set_variants(dnsp_poisson* h, int xvar, int zvar, int tvar);
