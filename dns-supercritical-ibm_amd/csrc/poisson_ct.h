@@ -274,8 +274,10 @@ __global__ __launch_bounds__(NT) void kt_xbwd(const double* S, double* P, long n
                                               const double2* __restrict__ tw, double scale, double* const* at) {
     __shared__ double2 sm[G * ct_pitch(N)];
     __shared__ double2 stw[N];
+    const double* const src = array_at<const double>(S, at);
+    double* const dst = array_at(P, at);
     ct_stage_twiddles<N, NT>(stw, tw);
-    xbwd_body<N, G, NT>(array_at<const double>(S, at), array_at(P, at), nlines, stw, scale, xcd_tile(blockIdx.x, gridDim.x), sm);
+    xbwd_body<N, G, NT>(src, dst, nlines, stw, scale, xcd_tile(blockIdx.x, gridDim.x), sm);
 }
 
 // ---------------------------------------------------------------------------
@@ -538,8 +540,9 @@ __global__ __launch_bounds__(NT) void kt_xfwd_xb(const double* P, double* W, lon
                                                  const double2* __restrict__ tw, const double* const* at) {
     __shared__ double2 sm[G * ct_pitch(N)];
     __shared__ double2 stw[N];
+    const double* const src = array_at(P, at);
     ct_stage_twiddles<N, NT>(stw, tw);
-    xfwd_body<N, G, NT, true>(array_at(P, at), W, nlines, stw, xcd_tile(blockIdx.x, gridDim.x), sm, nz);
+    xfwd_body<N, G, NT, true>(src, W, nlines, stw, xcd_tile(blockIdx.x, gridDim.x), sm, nz);
 }
 
 // z forward, XB -> MM.  Tile (k, c): the 16 x rows 16c..16c+15 of plane k as
