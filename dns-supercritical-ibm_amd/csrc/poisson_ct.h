@@ -39,7 +39,8 @@ __device__ __forceinline__ T* array_at(T* p, T* const* at) {
     return (T*)(GlobalPtr)(at ? *reinterpret_cast<const uintptr_t*>(at) : reinterpret_cast<uintptr_t>(p));
 }
 // The z transforms of 512 points keep ordinary loads: 384x512x256 takes 846 us with
-// them, 874 past the caches (z forward alone at 512x512x288 267 and 305).
+// them, 874 past the caches (z forward alone at 512x512x288 267 and 305).  A
+// measured exception: why this length differs from 384 and 768 is not known.
 constexpr bool z_loads_past(int n) { return n != 512; }
 
 // FFT kernel variants: (complex elements per workgroup tile, threads), one

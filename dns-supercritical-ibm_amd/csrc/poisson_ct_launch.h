@@ -48,7 +48,8 @@ const RgOps* rg_ops(int n);  // NULL where not supported
 // elements a workgroup where the field outgrows the 256 MB cache (768x384x384
 // 354 against 368 for 768, 256x256x256 43 against 46), else 768 (512x128x192 35
 // against 39).  Inverse: 768 at 384 and 512 points (384x384x256 100 against
-// 105), else 1536 (256x256x256 39 against 41, 768x384x384 316 against 321).
+// 105), else 1536 (256x256x256 39 against 41, 768x384x384 316 against 321):
+// measured by length, without a known cause.
 constexpr int blk_xfwd_variant(size_t points) { return points >= ((size_t)1 << 24) ? 2 : 0; }
 constexpr int blk_xbwd_variant(int nx) { return nx == 384 || nx == 512 ? 0 : 2; }
 constexpr int kBlkZVariant = 1;

@@ -33,7 +33,7 @@ struct dnsp_poisson {
     int xvar = 0, zvar = 0;           // their (tile, threads) variants, forward
     int xvar_b = 0, zvar_b = 0;       // and inverse transforms
     // blocked FP64 solve (x-blocked and mode-major layouts through d_W)
-    bool blk_ok = false;              // supported sizes (nx % 16 == 0, compile-time FFTs, partitioned)
+    bool blk_ok = false;              // supported sizes (compile-time FFTs, partitioned)
     bool blk_on = true;               // used by dnsp_poisson_run / solve when supported
     double* d_W = nullptr;            // its workspace, nx*nz*ny doubles
     int bxvar = 0, bxvar_b = 2;       // its x variants (forward, inverse)

@@ -151,7 +151,8 @@ int dnsp_poisson_stage(dnsp_poisson* h, const double* src, double* P, int stage,
 
 /* Kernel strategy (also the knobs of the tuner):
  *   fft:     DNSP_FFT_AUTO (compile-time-sized kernels where the length has
- *            them, else the runtime-sized ones), DNSP_FFT_GENERIC (always the
+ *            them, else the register-direct ones for lengths 16..768, else
+ *            the runtime-sized ones), DNSP_FFT_GENERIC (always the
  *            runtime-sized kernels), DNSP_FFT_FIXED (compile-time-sized only;
  *            DNSP_ERR_UNSUPPORTED if a length has none)
  *   tridiag: DNSP_TRIDIAG_AUTO (partitioned for ny >= 32), DNSP_TRIDIAG_SERIAL
@@ -184,10 +185,10 @@ int dnsp_poisson_get_strategy(const dnsp_poisson* h, int* fft_ct_x, int* fft_ct_
  * (2), (16, 16) for ny <= 512, else (64, 8) (3); rows per chunk follow from ny.
  * 4, 5, 7: the shapes of 0, 1, 3 with two-pass chunks (the chunk interior is
  * solved again once its end values are known, instead of being kept in
- * registers across the reduced solve); 6: as 2.  A handle starts with 2.  The mixed-precision
- * form has its own set; on its FP32 spectra shape 2 has twice the modes
- * (32, and 16 above 512 rows), 3 and 7 are (16, 32): 32 modes make 128-byte
- * rows.  No counterpart in the reference. */
+ * registers across the reduced solve); 6: as 2.  A handle starts with 2.  The
+ * mixed-precision form has its own set; on its FP32 spectra shape 2 has twice
+ * the modes (32, and 16 above 512 rows), 3 and 7 are (16, 32): 32 modes make
+ * 128-byte rows.  No counterpart in the reference. */
 int dnsp_poisson_set_variants(dnsp_poisson* h, int xvar, int zvar, int tvar);
 int dnsp_poisson_get_variants(const dnsp_poisson* h, int* xvar, int* zvar, int* tvar);
 int dnsp_poisson_set_mixed_variants(dnsp_poisson* h, int xvar, int zvar, int tvar);
@@ -197,7 +198,8 @@ int dnsp_poisson_get_mixed_variants(const dnsp_poisson* h, int* xvar, int* zvar,
  * of each direction, and pairs of tridiagonal solves of every partitioned
  * variant, on `work` (nx*nz*ny device doubles, overwritten; NULL = a
  * temporary allocation) and keeps the fastest in the handle; for a
- * DNSP_PRECISION_MIXED handle the same for the mixed-precision kernels.
+ * DNSP_PRECISION_MIXED handle the same for the mixed-precision kernels.  A
+ * `work` that is not 16-byte aligned times no x and no blocked-solve kernels.
  * times_ms (optional, DNSP_TUNE_SLOTS doubles) receives the mean ms per pair:
  * 4 x, 4 z and 8 tridiagonal variants of the FP64 form (slots 0..15), then
  * the same of the mixed form (16..31); -1 where not applicable.  Synchronises
